@@ -763,7 +763,6 @@ static int launch(ft_schedule *S, int precision, int kind, int dir, void *dA, vo
         if (dA) b.A = dA;  /* batches keep their own base */
         int spin = KNOB_GET(g_spin_limit);
         b.spin_limit = spin ? spin : 1 << 22;
-        b.trace = NULL;
         return ftamd_hip_sys_launch(&b, precision, S->L, stream);
     }
     FtamdLaunch a = S->launch;

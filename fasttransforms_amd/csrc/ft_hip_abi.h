@@ -160,7 +160,6 @@ typedef struct {
     int *prog;        /* [nprog] rows published by each split part, zero at launch; reset by the kernel */
     int nprog;
     int spin_limit;   /* polls before a wait gives up (FTAMD_ERR_TIMEOUT) */
-    unsigned long long *trace;  /* diagnostic per-wave timeline (instrumented builds only), else NULL */
 } FtamdSysLaunch;
 
 int ftamd_hip_sys_launch(const FtamdSysLaunch *a, int precision, int S, void *stream);

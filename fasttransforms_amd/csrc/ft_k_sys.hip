@@ -2,9 +2,9 @@
 // its C-ABI launcher.
 #include "ft_systolic.hpp"
 
-// S = 4 in FP64 does not fit the 128 VGPRs a 16-wave workgroup allows
-// without spilling; those plans run on the pipelined engine.
-extern "C" int ftamd_hip_sys_supported(int S, int precision) { return S == 2 || (S == 4 && precision == 1); }
+// Two sequences a lane: four in FP64 do not fit the 128 VGPRs a 16-wave
+// workgroup allows without spilling.
+extern "C" int ftamd_hip_sys_supported(int S, int precision) { return S == 2 && (precision == 0 || precision == 1); }
 
 extern "C" int ftamd_hip_sys_launch(const FtamdSysLaunch *a, int precision, int S, void *stream) {
     using Fn = void (*)(FtamdSysLaunch);
@@ -14,8 +14,7 @@ extern "C" int ftamd_hip_sys_launch(const FtamdSysLaunch *a, int precision, int 
     // (one mask per lane row); tri chains have one order per column
     const bool rm = a->rowmask != 0;
     if (precision == 0) fn = rm ? ftsys::sys_kernel<double, 2, true> : ftsys::sys_kernel<double, 2, false>;
-    else if (S == 2) fn = rm ? ftsys::sys_kernel<float, 2, true> : ftsys::sys_kernel<float, 2, false>;
-    else if (S == 4) fn = rm ? ftsys::sys_kernel<float, 4, true> : ftsys::sys_kernel<float, 4, false>;
+    else fn = rm ? ftsys::sys_kernel<float, 2, true> : ftsys::sys_kernel<float, 2, false>;
     if (!fn) return FTAMD_EINVAL;
     if (a->nchains <= 0) return FTAMD_OK;
     // the kernel indexes xcd_slot[0 .. nxcd] and one ticket per XCD

@@ -62,16 +62,23 @@ constexpr int kLanes = FTAMD_SYS_LANES;
 constexpr int kRows = 4;
 constexpr int kCols = 2;
 constexpr int kWaves = FTAMD_SYS_WAVES;
-// ring positions between two bands (a multiple of kU, at least 2*kChunk):
+// ring slots between two bands (a multiple of kU):
 // 64 lets a band run up to 64 rows ahead of the next (64 KB of LDS per
 // workgroup; 3-9 % faster than 32 at n = 1024, 80 no better)
 constexpr int kZ = 64;
 constexpr int kU = FTAMD_SYS_UNROLL;   // steps per loop iteration
 constexpr int kDin = 2;                // input positions read ahead
-constexpr int kChunk = 16;             // matrix rows fetched per lane-parallel load
+constexpr int kChunk = 16;             // rows of another part fetched per lane-parallel load
 
 
 template <typename T> using Pair = T __attribute__((ext_vector_type(2)));
+
+// The launch's records never change while it runs: read through the constant
+// address space, so that wave-uniform reads are scalar loads.
+typedef __attribute__((address_space(4))) FtamdSysBand ConstBand;
+typedef __attribute__((address_space(4))) FtamdSysChain ConstChain;
+typedef __attribute__((address_space(4))) FtamdSysItem ConstItem;
+typedef __attribute__((address_space(4))) int ConstInt;
 
 __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
 
@@ -99,6 +106,11 @@ struct Engine {
     // S+1 steps per lane (the lane's S sequences pass it on within a step,
     // the DPP shift to the next lane takes a step)
     static constexpr int kOutDelay = (S + 1) * (kLanes - 1) + S;
+    // steps the table entries are read out of LDS ahead of their use
+    static constexpr int kAhead = 2;
+    // what a band has besides its neighbours' rings: rows from A all along (a
+    // chain's first band), rows to A all along (its last), either
+    static constexpr int kInner = 0, kFirst = 1, kLast = 2, kBoth = 3;
 
     // table bytes of one step (all 16 lanes) and steps per 1 KB LDS-DMA load
     static constexpr int kStepBytes = kLanes * S * 2 * (int)sizeof(T);
@@ -123,59 +135,41 @@ struct Engine {
         // a lane's S pairs in one 128-bit read); the tables are laid out
         // the same way (FTAMD_SYS_SLOT_MAJOR)
         Pair<T> scr[kWaves][kD][kLanes * S];
-        T ring[kWaves][kZ][kRows][kCols];  // ring g: input stream of the band wave g runs
-        int avail[kWaves];                 // positions of ring g written by wave g-1 (exclusive end)
-        int freed[kWaves];                 // positions of ring g wave g has read (exclusive end)
+        Pair<T> ring[kWaves][kZ][kRows];  // ring g: input stream of the band wave g runs (a row's two columns)
+        // per wave, published together after every block: the ring slots of
+        // ring g it has read, and those of ring g+1 it has written (exclusive ends)
+        struct Published {
+            int freed, avail;
+        } pub[kWaves + 2];                 // wave g's at index g + 1
+        Pair<T> ident[kD][kLanes * S];     // (0, 1): what a masked sequence reads in place of scr
+        unsigned spare[64];                // where fillers go
         int abort_flag;
         int slot;                          // the workgroup's current slot (ticket)
     };
 
-    // The table entries of one lane for one step: S (s, c) pairs.
-    struct SC {
-        Pair<T> p[S];
-        __device__ Pair<T> pair(int s) const { return p[s]; }
+    // The table entries of one lane for one step: S (s, c) pairs, one for each
+    // of MC columns or one for both.
+    template <int MC> struct SC {
+        Pair<T> p[S][MC];
     };
 
     // A wave whose wait expires raises the workgroup's abort flag (every
     // other wait then ends too) and reports the error once its loop is left.
     __device__ static void fail(Shared &sh) { lds_st(&sh.abort_flag, 1); }
 
-#ifdef FTAMD_TRACE
-    // per-wave accumulators of wait clocks (instrumented builds)
-    __device__ static unsigned long long &tr_in() {
-        static __shared__ unsigned long long v[kWaves];
-        return v[threadIdx.x >> 6];
-    }
-    __device__ static unsigned long long &tr_out() {
-        static __shared__ unsigned long long v[kWaves];
-        return v[threadIdx.x >> 6];
-    }
-    __device__ static unsigned long long &tr_dma() {
-        static __shared__ unsigned long long v[kWaves];
-        return v[threadIdx.x >> 6];
-    }
-#endif
 
-    // Waits until *ctr >= need (seen caches the last value read), at most
-    // `limit` polls.
+    // Waits until *ctr >= need (seen: the last value read), at most `limit`
+    // polls.
     __device__ static bool wait_ge(Shared &sh, int *ctr, int need, int &seen, int limit) {
-#ifdef FTAMD_TRACE
-        struct Acc {
-            unsigned long long t0, *dst;
-            __device__ ~Acc() {
-                if ((threadIdx.x & 63) == 0) *dst += __builtin_amdgcn_s_memtime() - t0;
-            }
-        } acc{__builtin_amdgcn_s_memtime(), (ctr >= &sh.avail[0] && ctr < &sh.avail[kWaves]) ? &tr_in() : &tr_out()};
-#endif
-        for (int it = 0; seen < need; ++it) {
+        for (int it = 1;; ++it) {
+            seen = uniform(lds_ld(ctr));
+            if (seen >= need) return true;
             if (it >= limit || uniform(lds_ld(&sh.abort_flag))) return false;
             // far behind (a band waiting for the chain's fill): poll rarely,
             // so waiting waves leave the issue slots to the working ones
-            if (need - seen > 2 * kU) __builtin_amdgcn_s_sleep(16);
+            if (need - seen > 2 * kU) __builtin_amdgcn_s_sleep(4);
             else __builtin_amdgcn_s_sleep(1);
-            seen = uniform(lds_ld(ctr));
         }
-        return true;
     }
 
     // Table entries reach the waves by LDS DMA (global_load_lds_dwordx4: 64
@@ -201,45 +195,48 @@ struct Engine {
                      : "s"(uniform((int)lds)), "v"(lane16), "s"(src), "v"(after)
                      : "memory");
     }
-    // The same, with the step split into a uniform base and a compile-time
-    // part K: the instruction's immediate offset is added to both the global
-    // and the LDS address, so M0 stays at the base slot and offset:K*bytes
-    // selects step base+K on both sides.
+    // The same in the loop, with the step split into a uniform base and a
+    // compile-time part K: the instruction's immediate offset is added to both
+    // the global and the LDS address, so M0 stays at the base slot for a whole
+    // block of steps (set_m0) and offset:K*bytes selects step base+K on both
+    // sides.
+    __device__ static void set_m0(unsigned lds_base) { asm volatile("s_mov_b32 m0, %0" : : "s"(lds_base) : "memory"); }
     template <int K>
-    __device__ static void dma_block_at(unsigned lds_base, const char *src_base, unsigned lane16, T after) {
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%4"
+    __device__ static void dma_block_at(const char *src_base, unsigned lane16, T after) {
+        asm volatile("global_load_lds_dwordx4 %0, %1 offset:%3"
                      :
-                     : "s"(lds_base), "v"(lane16), "s"(src_base), "v"(after), "n"(K * kStepBytes)
+                     : "v"(lane16), "s"(src_base), "v"(after), "n"(K * kStepBytes)
                      : "memory");
     }
-    // Called before the first read of a block, one step before its first
+    // A DMA of a dword a lane from the start of the tables to nowhere in particular.
+    __device__ static void dma_filler(Shared &sh, const void *tab, unsigned lane16) {
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                     :
+                     : "s"(uniform((int)lds_addr(sh.spare))), "v"(lane16), "s"(tab)
+                     : "memory");
+    }
+    // Called before the first read of a block, kAhead steps before its first
     // step, when the two blocks after it have been requested and the third
     // not yet.
+    // `Extra`: other vector memory operations issued since the block that may
+    // stay outstanding with them.
+    template <int Extra = 0>
     __device__ static void wait_block() {
-#ifdef FTAMD_TRACE
-        const unsigned long long c0 = __builtin_amdgcn_s_memtime();
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kD / kSPD - 2) : "memory");
-        if ((threadIdx.x & 63) == 0) tr_dma() += __builtin_amdgcn_s_memtime() - c0;
-#else
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kD / kSPD - 2) : "memory");
-#endif
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kD / kSPD - 2 + Extra) : "memory");
     }
-    // Lane 15 of each row of 16 (the row's last sequence) to every lane of
-    // the row (DPP row_newbcast:15).
-    // (Every lane has a source, so the old value is irrelevant: one DPP move.)
-    __device__ static T row_end(T v) { return __builtin_amdgcn_update_dpp(T(0), v, 0x15f, 0xf, 0xf, true); }
+    // Lane 15 of each row of 16 (the row's last sequence), DPP row_newbcast:15,
+    // into the lanes 4b .. 4b+3 of each row (bank b) of `keep`.
+    template <int B> __device__ static T row_end(T keep, T v) {
+        return __builtin_amdgcn_update_dpp(keep, v, 0x15f, 0xf, 1 << B, false);
+    }
     __device__ static unsigned lds_addr(const void *p) { return (unsigned)(uintptr_t)p; }
+    template <typename V> using Lds = __attribute__((address_space(3))) V;
+    template <typename V> __device__ static Lds<V> *lds_at(unsigned addr) { return (Lds<V> *)(uintptr_t)addr; }
 
     // position of (lane i, slot s) in a step's entries, and of lane i's first
     static constexpr bool kSlotMajor = sizeof(T) == 8;
     static constexpr int kSlotStride = kSlotMajor ? kLanes : 1;
     __device__ static int lane_entry(int i) { return kSlotMajor ? i : i * S; }
-
-    __device__ static void read_sc(Shared &sh, int w, int step, int i, SC &sc) {
-        const Pair<T> *p = &sh.scr[w][step % kD][lane_entry(i)];
-#pragma unroll
-        for (int s = 0; s < S; ++s) sc.p[s] = p[s * kSlotStride];
-    }
 
     // Progress counters of split chains.  The producing band stores its rows
     // to A with device-scope stores and, once they are complete, publishes
@@ -262,60 +259,86 @@ struct Engine {
         return true;
     }
 
-    // One step: rotate every (sequence, column) of the lane.  X0: the fresh
-    // rows of the lane's first sequence (the last sequence of the lane before
-    // emitted them at the previous step, or the stream at lane 0); Y: carried
-    // rows; sequence s > 0 takes as its fresh row what sequence s-1 emits in
-    // this step.
-    // MASK 0: every column applies every sequence of the band; 1: the two
-    // columns of a lane row apply the same sequences (mask [s][0]); 2: per
-    // column.  A sequence a column does not apply is the identity (0, 1):
-    // with m = 1 where the column applies the sequence and 0 where not, the
-    // applied pair is (s*m, fma(c, m, 1-m)), exact for both values of m and
-    // two FP64 operations where a select of two doubles takes four.
-    template <int MASK>
-    __device__ static void rotate(T (&Y)[S][kCols], T (&E)[S][kCols], const T (&X0)[kCols], const SC &sc,
-                                  const T (&m)[S][kCols], const T (&m1)[S][kCols]) {
+    // One step in two halves, so that what the next lane and the next step
+    // wait for comes first: emit() computes every sequence's outgoing row,
+    // carry() its new carried row, after the step's LDS accesses are issued.
+    // X0: the fresh rows of the lane's first sequence (the last sequence of
+    // the lane before emitted them at the previous step, or the stream at
+    // lane 0); Y: carried rows; sequence s > 0 takes as its fresh row what
+    // sequence s-1 emits in this step.
+    template <int MC> struct Applied {  // a step's (s, c) with its fresh rows
+        SC<MC> sc;
+        T x[S][kCols];
+    };
+    template <int MC>
+    __device__ static void emit(const T (&Y)[S][kCols], T (&E)[S][kCols], const T (&X0)[kCols], const SC<MC> &sc,
+                                Applied<MC> &ap) {
+        ap.sc = sc;
 #pragma unroll
-        for (int s = 0; s < S; ++s) {
-            const Pair<T> e = sc.pair(s);
-            const T sn_row = MASK == 1 ? e.x * m[s][0] : e.x;
-            const T cs_row = MASK == 1 ? fmaT<T>(e.y, m[s][0], m1[s][0]) : e.y;
+        for (int s = 0; s < S; ++s)
 #pragma unroll
             for (int c = 0; c < kCols; ++c) {
-                const T x = s == 0 ? X0[c] : E[s - 1][c];
-                const T y = Y[s][c];
-                T sn = sn_row, cs = cs_row;
-                if (MASK == 2) {
-                    sn = e.x * m[s][c];
-                    cs = fmaT<T>(e.y, m[s][c], m1[s][c]);
-                }
-                Y[s][c] = fmaT<T>(cs, x, sn * y);
-                E[s][c] = fmaT<T>(cs, y, -(sn * x));
+                const Pair<T> e = sc.p[s][c % MC];
+                ap.x[s][c] = s == 0 ? X0[c] : E[s - 1][c];
+                E[s][c] = fmaT<T>(e.y, Y[s][c], -(e.x * ap.x[s][c]));
             }
-        }
+    }
+    template <int MC> __device__ static void carry(T (&Y)[S][kCols], const Applied<MC> &ap) {
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int c = 0; c < kCols; ++c) {
+                const Pair<T> e = ap.sc.p[s][c % MC];
+                Y[s][c] = fmaT<T>(e.y, ap.x[s][c], e.x * Y[s][c]);
+            }
     }
 
-    // w: the band's index in its chain; g: the wave (and ring) index in the
-    // workgroup.  Ring positions are counted across the chains a workgroup
-    // streams: this band's input stream starts at position in_base of ring g,
-    // its output (the next band's input) at out_base of ring g+1, both
-    // multiples of kZ.  LINK: the band hands rows to or takes them from
-    // another part of its chain (through A).  Returns false if a wait expired
-    // (abort raised).
-    template <int MASK, bool LINK>
-    __device__ static bool run_band(const FtamdSysLaunch &a, Shared &sh, const FtamdSysChain &ch, int w, int g,
-                                    int lane, int in_base, int out_base) {
+    // w: the band's index in its chain part; g: the wave (and ring) index in
+    // the workgroup.  Ring slots are counted across the chains a workgroup
+    // streams: this band's input stream starts at slot in_base of ring g, its
+    // output (the next band's input) at out_base of ring g+1, both multiples
+    // of kZ; stream position p is in slot off + p (idle()).  END: kFirst a
+    // chain's first band, kLast its last, kBoth any; MASK 0: every column
+    // applies every sequence of the band; 1: the two columns of a lane row
+    // apply the same sequences; 2: per column (a sequence a column does not
+    // apply is the identity (0, 1), read from a block of identities in place
+    // of the table: no arithmetic); LINK: a band that hands
+    // rows to or takes them from another part of its chain (through A).
+    // Returns false if a wait expired (abort raised).
+    //
+    // What bounds it: a step is 16 FP64 operations (S = 2), 4 DPP moves to the
+    // next lane and 2 that keep its outputs; an LDS write takes 13 clocks of
+    // the CU's LDS input whatever its lane mask (a 128-bit read 4), so
+    // outputs are kept in registers and leave a block of 8 at a time: the DPP
+    // broadcast of the row's last lane writes one bank of 4 lanes per step
+    // under its bank mask, no selects.  A step's outputs are kept a step late,
+    // which takes them off the critical path.  Everything
+    // that does not happen in every block waits for a step count (t_in, t_out):
+    // a block's own work is one compare, its steps, its outputs and one write
+    // of the counters.  (sph hi2lo n = 1024, 1024 x 2047 FP64, with the copy
+    // of the coefficients before it: 170 -> 142 us; FP32 lo2hi n = 733: 89 ->
+    // 67 us, against selects per step, an LDS round trip per wait and the
+    // first band's rows through registers.  A step takes a lone wave about 190
+    // clocks, 22 of its instructions on the vector ALU; with four waves on a
+    // SIMD the ALU bounds it.)
+    template <int MASK, int END, bool LINK>
+    __device__ static bool run_band(const FtamdSysLaunch &a, Shared &sh, const ConstChain &ch, const FtamdSysChain &cv,
+                                    int w, int g, int lane, int in_base, int out_base) {
+        constexpr int kLag = kOutDelay + 1;  // a position's steps from lane 0 to its store
+        constexpr int kNever = 0x7fffffff;
+        // what follows from the lane is computed here, not once for every
+        // instantiation before the loop over the parts (it would not fit the
+        // registers)
+        asm volatile("" : "+v"(lane));
         const int r = lane >> 4, i = lane & 15;
         const int nb = uniform(ch.nb);
-        const int b = uniform(ch.band0) + w;
-        const int R = uniform(a.bands[b].R);
-        const int steps = uniform(a.bands[b].steps);
-        const int gbase = uniform(a.bands[b].gbase);
-        const bool first = w == 0, last = w == nb - 1;
+        const ConstBand *band = (const ConstBand *)(uintptr_t)a.bands + (uniform(ch.band0) + w);
+        const int R = uniform(band->R);
+        const int gbase = uniform(band->gbase);
+        const bool first = END == kBoth ? w == 0 : END == kFirst, last = END == kBoth ? w == nb - 1 : END == kLast;
         const int dir = uniform(ch.dir);
-        const int Rprev = first ? 0 : uniform(a.bands[b - 1].R);
-        const int Rnext = last ? -1 : uniform(a.bands[b + 1].R);
+        const int Rprev = first ? 0 : uniform(band[-1].R);
+        const int off = idle(w);
         // stream positions 0 .. npa-1 come from A, the rest from the previous band
         const int npa = first ? R + 1 : (dir == 0 ? R - Rprev : 0);
         // a part after the first of its chain: its positions from npa_own on
@@ -324,291 +347,368 @@ struct Engine {
         // every row it emits and publishes them on counter split_out
         const int split_in = LINK && first ? uniform(ch.split_in) : -1;
         const int split_out = LINK && last ? uniform(ch.split_out) : -1;
-        const int npa_own = split_in >= 0 && dir == 0 ? R - uniform(a.bands[b - 1].R) : 0;
+        const bool polled = LINK && split_in >= 0;
+        const int npa_own = polled && dir == 0 ? R - uniform(band[-1].R) : 0;
         int prog_seen = 0, published = 0, pub = 0;
-        // the next band's position of our output position p is p + npa_next;
-        // outputs beyond the next band's stream leave the chain
-        const int npa_next = last ? 0 : (dir == 0 ? Rnext - R : 0);
-        const int rstep = uniform(ch.rstep), rpar = uniform(ch.rpar);
-        const long long lda = uniform(ch.lda);
+        // output position p goes to slot p + out_off of the next band's
+        // stream; positions beyond ring_hi leave the chain (or the part)
+        int ring_hi = -1, out_off = 0;
+        if (!last) {
+            const int Rnext = uniform(band[1].R);
+            const int npa_next = dir == 0 ? Rnext - R : 0;
+            ring_hi = min(R, Rnext - npa_next);
+            out_off = npa_next + idle(w + 1);
+        }
+        const long long rstep = uniform(ch.rstep), lda = uniform(ch.lda);
+        const int rpar = uniform(ch.rpar);
         const int spin = uniform(a.spin_limit);  // polls before a wait gives up
         T *A = (T *)a.A + ch.aoff;
-        const int colv[kCols] = {ch.col[2 * r], ch.col[2 * r + 1]};
-        const char *tab_band = (const char *)a.tab + a.bands[b].tab * (long long)sizeof(Pair<T>);
+        // step t takes the table's step t - off (the steps before a later
+        // band's table are the spare steps of the band before: identities)
+        const char *tab_band = (const char *)a.tab + (band->tab * (long long)sizeof(Pair<T>) - (long long)off * kStepBytes);
         const unsigned lane16 = (unsigned)lane * 16u;
-
-        // matrix element of class row e of column c of this lane's row
-        auto aptr = [&](int c, int e) -> T * { return A + (long long)colv[c] * lda + (long long)rstep * e + rpar; };
-        // class row of stream position p
-        auto row_of = [&](int p) { return dir == 0 ? R - p : p; };
-
-        // with MASK 1 column 0 of a row carries the row's mask (column 1's
-        // when column 0 is absent)
-        T m[S][kCols], m1[S][kCols];
-#pragma unroll
-        for (int s = 0; s < S; ++s)
-#pragma unroll
-            for (int c = 0; c < kCols; ++c) {
-                const int q = gbase + S * i + s;
-                const int k = MASK == 1 && c == 0 && colv[0] < 0 ? 2 * r + 1 : 2 * r + c;
-                const bool on = q >= ch.glo[k] && q <= ch.ghi[k];
-                m[s][c] = on ? T(1) : T(0);
-                m1[s][c] = on ? T(0) : T(1);
-            }
-
-        T(*in_ring)[kRows][kCols] = sh.ring[g];
-        T(*out_ring)[kRows][kCols] = last ? sh.ring[g] : sh.ring[g + 1];
-        int avail_seen = 0, freed_seen = 0;  // last counter values read (global positions)
-        bool ok = true;
-#ifdef FTAMD_TRACE
-        if (lane == 0) tr_in() = tr_out() = tr_dma() = 0;
-        const unsigned long long tr_start = wall_clock64(), tr_c0 = __builtin_amdgcn_s_memtime();
-#endif
-
-        // ---- stream positions from A: lane i of each row fetches position
-        // p0 + i of a chunk of 16.  (Loads and stores of A only make the
-        // waits on the table loads stricter: see the output stores.)
-        auto fetch = [&](int p0, T (&v)[kCols]) -> bool {
-            const int p = p0 + i;
-            if (split_in >= 0) {
-                const int need = min(p0 + kChunk - 1, R) - npa_own + 1;
-                if (need > 0 && !wait_prog(sh, a.prog + split_in, need, prog_seen, spin)) return false;
-#pragma unroll
-                for (int c = 0; c < kCols; ++c)
-                    v[c] = (p <= R && colv[c] >= 0)
-                               ? __hip_atomic_load(aptr(c, row_of(p)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                               : T(0);
-                return true;
-            }
-#pragma unroll
-            for (int c = 0; c < kCols; ++c)
-                v[c] = (p < npa && p <= R && colv[c] >= 0) ? *aptr(c, row_of(p)) : T(0);
-            return true;
-        };
-        auto put = [&](int p0, const T (&v)[kCols]) {
-            const int p = p0 + i;
-            if (p < npa) {
-#pragma unroll
-                for (int c = 0; c < kCols; ++c) lds_st(&in_ring[p % kZ][r][c], v[c]);
-            }
-        };
-        // chunk k (positions 16k .. 16k+15) is fetched 16 steps before it is
-        // written to the ring, 32 steps before it is read
-        T chunk[kCols];
-        {
-            T v[kCols];
-            ok = fetch(0, v);
-            put(0, v);
-            ok = ok && fetch(kChunk, chunk);
-        }
-
-        // ---- input prefetch: positions 0 .. kDin-1
-        T inbuf[kDin][kCols];
-        auto ensure_in = [&](int p) -> bool {
-            bool good = true;
-            if (p >= npa && p <= R && in_base + p >= avail_seen)
-                good = wait_ge(sh, &sh.avail[g], in_base + p + 1, avail_seen, spin);
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            return good;
-        };
-        auto read_in = [&](int p, T (&v)[kCols]) {
-#pragma unroll
-            for (int c = 0; c < kCols; ++c) v[c] = lds_ld(&in_ring[p % kZ][r][c]);
-        };
-#pragma unroll
-        for (int d = 0; d < kDin; ++d) {
-            ok = ok && ensure_in(d);
-            read_in(d, inbuf[d]);
-        }
 
         // ---- table prefetch: steps 0 .. kD-1
 #pragma unroll
         for (int d = 0; d < kD; d += kSPD) dma_block(sh, g, tab_band, d, lane16, T(0));
 
-        T Y[S][kCols], E[S][kCols];
+        // class row of stream position p
+        auto row_of = [&](int p) { return dir == 0 ? R - p : p; };
+        const long long astep = dir == 0 ? -rstep : rstep;  // elements of A from one position to the next
+
+        Pair<T>(*in_ring)[kRows] = sh.ring[g];
+        T *out_ring = (T *)sh.ring[last ? g : g + 1];
+        int *const avail = &sh.pub[g].avail;       // of the wave before
+        int *const freed = &sh.pub[g + 2].freed;   // of the wave after
+        const int slots = R + off;                 // the stream's last slot
+        bool ok = true;
+        // the slots before position 0 pass through as rows of zeros
+        if (i < off) in_ring[i][r] = Pair<T>{T(0), T(0)};
+
+        // ---- stream positions from A.  By LDS DMA straight into the ring: a
+        // load of one dword a lane covers kRowsDma positions (8 elements each,
+        // in the ring's order), so no register waits for it, and the waits on
+        // the table DMAs issued after it cover it.
+        constexpr int kDw = (int)sizeof(T) / 4;
+        constexpr int kRowsDma = 64 / (FTAMD_SYS_COLS * kDw);  // positions of one DMA
+        const int de = lane / kDw;                              // the lane's element of the block
+        const int dcol = cv.col[de % FTAMD_SYS_COLS], dpos = de / FTAMD_SYS_COLS;
+        const char *rows_src = (const char *)(A + ((long long)max(dcol, 0) * lda + rpar + rstep * row_of(dpos))) +
+                               4 * (lane % kDw);
+        const unsigned in_lds = uniform(lds_addr(in_ring));
+        const unsigned long long rows_on = __ballot(dcol >= 0);
+        auto dma_rows = [&](int p0) {  // positions p0 .. p0 + kRowsDma - 1 (those below npa)
+            unsigned long long on = rows_on;
+            if (p0 + kRowsDma > npa) on = __ballot(dcol >= 0 && p0 + dpos < npa);
+            unsigned long long save;
+            asm volatile("s_mov_b64 %0, exec\n\ts_mov_b32 m0, %1\n\ts_mov_b64 exec, %2\n\t"
+                         "global_load_lds_dword %3, off\n\ts_mov_b64 exec, %0"
+                         : "=&s"(save)
+                         : "s"(in_lds + (unsigned)((p0 + off) % kZ) * (unsigned)sizeof(Pair<T>[kRows])), "s"(on),
+                           "v"(rows_src)
+                         : "memory");
+            rows_src += astep * (kRowsDma * (int)sizeof(T));
+        };
+        // how far ahead of the step that starts a block its rows are requested
+        constexpr int kRowsAhead = 32;
+        // A band that takes rows from A all along or stores its rows there
+        // issues this many vector memory operations per block after its last
+        // table DMA and before the next block's first: the next rows from A,
+        // a store of A, or a filler in their place, so that the waits on the
+        // table DMAs can leave them outstanding (rows of A take a trip to HBM).
+        constexpr int kExtra = (END & kFirst ? kU / kRowsDma : 0) + (END & kLast ? 1 : 0);
+        static_assert(kZ >= kRowsAhead + 2 * kU, "slots are read before they are written again");
+
+        // A chain part that takes rows from another part polls for them and
+        // reads them with device-scope loads: lane i of each row fetches
+        // position p0 + i of a chunk of 16, 16 steps before it is written to
+        // the ring, 32 before it is read.
+        const int colv[kCols] = {cv.col[2 * r], cv.col[2 * r + 1]};
+        auto aptr = [&](int c, int e) -> T * { return A + ((long long)colv[c] * lda + rstep * e + rpar); };
+        T chunk[kCols] = {T(0), T(0)};
+        auto fetch = [&](int p0, T (&v)[kCols]) -> bool {
+            const int p = p0 + i;
+            const int need = min(p0 + kChunk - 1, R) - npa_own + 1;
+            if (need > 0 && !wait_prog(sh, a.prog + split_in, need, prog_seen, spin)) return false;
+#pragma unroll
+            for (int c = 0; c < kCols; ++c)
+                v[c] = (p <= R && colv[c] >= 0)
+                           ? __hip_atomic_load(aptr(c, row_of(p)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                           : T(0);
+            return true;
+        };
+        auto put = [&](int p0, const T (&v)[kCols]) {
+            const int p = p0 + i;
+            if (p <= R) in_ring[(p + off) % kZ][r] = Pair<T>{v[0], v[1]};
+        };
+
+        if (polled) {
+            T v[kCols];
+            ok = fetch(0, v);
+            put(0, v);
+            ok = ok && fetch(kChunk, chunk);
+        } else {
+            // (a band after the first takes at most B positions from A)
+            const int n0 = first ? min(npa, kRowsAhead) : npa;
+            for (int p = 0; p < n0; p += kRowsDma) dma_rows(p);
+        }
+
+        // where the lane reads the entries of sequence s for column c: with
+        // MASK 1 column 0 of a row carries the row's mask (column 1's when
+        // column 0 is absent)
+        constexpr int MC = MASK == 2 ? kCols : 1;
+        unsigned sc_at[S][MC];
 #pragma unroll
         for (int s = 0; s < S; ++s)
 #pragma unroll
-            for (int c = 0; c < kCols; ++c) Y[s][c] = E[s][c] = T(0);
-
-        // entries of step 0 (read one step ahead from here on)
-        SC scn;
-        wait_block();
-        read_sc(sh, g, 0, i, scn);
-
-        // Steps run in blocks of kU.  The waits are made once per block, so
-        // a step is only its DPP shifts, LDS reads, rotations and the
-        // broadcast of its output.
-        int written = out_base;  // ring positions of the next band written (exclusive end, global)
-        for (int t0 = 0; t0 < steps; t0 += kU) {
-            if (t0 % kChunk == 0) {
-                // positions t0+16 .. t0+31 to the ring, into the slots of
-                // positions t0+16-kZ .. t0+31-kZ (all read: kZ >= 32);
-                // fetch the next 16
-                const int p0 = t0 + kChunk;
-                if (p0 < npa) {
-                    put(p0, chunk);
-                    if (!fetch(p0 + kChunk, chunk)) {
-                        ok = false;
-                        break;
-                    }
-                }
+            for (int c = 0; c < MC; ++c) {
+                const int q = gbase + S * i + s;
+                const int k = MASK == 1 && colv[0] < 0 ? 2 * r + 1 : 2 * r + c;
+                const bool on = MASK == 0 || (q >= cv.glo[k] && q <= cv.ghi[k]);
+                sc_at[s][c] = lds_addr(on ? &sh.scr[g][0][0] : &sh.ident[0][0]) +
+                              (unsigned)(lane_entry(i) + s * kSlotStride) * (unsigned)sizeof(Pair<T>);
             }
-            // every input position the block reads ahead is in the ring
-            {
-                const int pl = min(t0 + kU - 1 + kDin, R);
-                if (pl >= npa && in_base + pl >= avail_seen &&
-                    !wait_ge(sh, &sh.avail[g], in_base + pl + 1, avail_seen, spin)) {
-                    ok = false;
-                    break;
+        auto read_sc = [&](int slot, SC<MC> &sc, unsigned at = 0) {
+#pragma unroll
+            for (int s = 0; s < S; ++s)
+#pragma unroll
+                for (int c = 0; c < MC; ++c) {
+                    // (MASK 0: one address, the slots by constant offsets)
+                    const Lds<Pair<T>> *q = MASK == 0 ? lds_at<Pair<T>>(sc_at[0][0] + at) + s * kSlotStride
+                                                   : lds_at<Pair<T>>(sc_at[s][c] + at);
+                    sc.p[s][c] = q[slot * kLanes * S];
                 }
-                __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        };
+
+        // ---- a block's outputs: lane i of each row holds output u =
+        // i / 4 + 4 (i % 2) of column (i / 2) % 2
+        const int out_u = (i >> 2) + 4 * (i & 1), out_c = (i >> 1) & 1;
+        const int ocol = out_c ? colv[1] : colv[0];
+        T outv[2][kCols];
+#pragma unroll
+        for (int c = 0; c < kCols; ++c) outv[0][c] = outv[1][c] = T(0);
+        // its row of A in the block that starts at step 0
+        T *out_a = A + ((long long)max(ocol, 0) * lda + rpar + rstep * row_of(0) + astep * (out_u - kLag - off));
+        const unsigned out_lane = lds_addr(out_ring) + (unsigned)(r * kCols + out_c) * (unsigned)sizeof(T);
+
+        // ---- the events between blocks: input slots the next block reads
+        // ahead must be in the ring, slots its outputs go to read by the next
+        // band, or (LINK) another part's rows read from A.
+        int avail_seen = 0, freed_seen = 0;  // last counter values read (global slots)
+        int t_chunk = polled && kChunk <= R ? 0 : kNever;                // next chunk of another part's rows
+        auto in_event = [&]() {  // first block that needs more than the slots known to be there
+            const int have = max(npa + off, avail_seen - in_base);
+            return have > slots ? kNever : have - (kU - 1 + kDin);
+        };
+        auto out_event = [&]() {  // first block whose outputs need more than the slots known to be free
+            const int have = freed_seen - out_base + kZ - out_off;  // positions below this may be written
+            return last || have > ring_hi ? kNever : max(have + kLag + off - (kU - 1), kLag);
+        };
+        int t_in = in_event(), t_out = out_event();
+        auto event = [&](int t0) -> bool {
+            if (LINK && t0 >= t_chunk) {
+                put(t0 + kChunk, chunk);
+                if (!fetch(t0 + 2 * kChunk, chunk)) return false;
+                t_chunk = t0 + 2 * kChunk <= R ? t0 + kChunk : kNever;
             }
-            // the block's outputs, positions po0 .. po0+kU-1: those in
-            // [0, R] go to the next band's ring up to position ring_hi,
-            // beyond it (or from the last band) they leave the chain
-            const int po0 = t0 - kOutDelay;
-            const int ring_hi = last ? -1 : min(R, Rnext - npa_next);
-            {
-                const int hi = min(po0 + kU - 1, ring_hi);
-                if (hi >= max(po0, 0)) {
-                    const int P1 = out_base + hi + npa_next;
-                    if (P1 - kZ >= freed_seen && !wait_ge(sh, &sh.freed[g + 1], P1 - kZ + 1, freed_seen, spin)) {
-                        ok = false;
-                        break;
+            if (t0 >= t_in) {
+                if (!wait_ge(sh, avail, in_base + min(t0 + kU - 1 + kDin, slots) + 1, avail_seen, spin)) return false;
+                t_in = in_event();
+            }
+            if (t0 >= t_out) {
+                if (!wait_ge(sh, freed, out_base + min(t0 - kLag - off + kU - 1, ring_hi) + out_off - kZ + 1, freed_seen, spin))
+                    return false;
+                t_out = out_event();
+            }
+            return true;
+        };
+
+        // ---- input prefetch: slots 0 .. kDin-1, table entries of steps 0 ..
+        // kAhead-1; the DMAs of the first rows are waited for here
+        Pair<T> inbuf[kDin];
+        SC<MC> scn[kAhead];
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        if (ok && min(kDin - 1, slots) >= npa + off)
+            ok = wait_ge(sh, avail, in_base + min(kDin - 1, slots) + 1, avail_seen, spin);
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int d = 0; d < kDin; ++d) inbuf[d] = in_ring[d][r];
+#pragma unroll
+        for (int d = 0; d < kAhead; ++d) read_sc(d, scn[d]);
+
+        T Y[S][kCols], E[S][kCols];
+        Applied<MC> ap;  // the step before's: Y = 0 * 0 + 0 * Y at first
+#pragma unroll
+        for (int s = 0; s < S; ++s)
+#pragma unroll
+            for (int c = 0; c < kCols; ++c) {
+                Y[s][c] = E[s][c] = ap.x[s][c] = T(0);
+                ap.sc.p[s][c % MC] = Pair<T>{T(0), T(0)};
+            }
+
+        const unsigned m0_base = uniform(lds_addr(&sh.scr[g][0][0]));
+        const int total = (slots + kLag + kU) & ~(kU - 1);  // the last position is stored in step slots + kLag
+        const int in_free_end = in_base + span(R, off);
+        constexpr unsigned kSlotBytes = sizeof(Pair<T>[kRows]);
+        const unsigned in_lane = in_lds + (unsigned)r * (unsigned)sizeof(Pair<T>);
+        const unsigned pub_lds = lds_addr(&sh.pub[g + 1]);
+        // the blocks whose outputs all go to the next band's ring, or (of a
+        // chain's last band) all to A: steps t_same .. t_same + n_same - 1
+        const int t_same = (kLag + off + kU - 1) & ~(kU - 1);
+        const int n_same = max(0, ((last ? R : ring_hi) + 1 + kLag + off - t_same) & ~(kU - 1));
+        const unsigned out_slot0 = (unsigned)(out_off - kLag - off + out_u);  // slot of the lane's output, less t0
+        const bool out_on = ocol >= 0;
+        int pub_freed = in_base, pub_avail = out_base;
+        unsigned pin = in_lane;                        // ring slot of position t0
+        asm volatile("" : "+v"(pin));
+
+        // Steps run in blocks of kU.
+        for (int t0 = 0, t_event = 0;;) {
+            if (t0 >= t_event) {
+                if (t0 >= total) break;
+                if (!ok || !event(t0)) {
+                    fail(sh);
+                    atomicOr(a.ctl + FTAMD_SYS_CTL_ERR, FTAMD_ERR_TIMEOUT);
+                    return false;
+                }
+                t_event = min(min(t_in, t_out), LINK ? min(t_chunk, total) : total);
+            }
+            if (END & kFirst) {
+                // the block's share of the rows from A (see kExtra)
+                const int p0 = t0 + kRowsAhead;
+                if (first && !polled && p0 < npa) {
+#pragma unroll
+                    for (int q = 0; q < kU; q += kRowsDma) {
+                        if (q == 0 || p0 + q < npa) dma_rows(p0 + q);
+                        else dma_filler(sh, a.tab, lane16);
                     }
-                    written = P1 + 1;
+                } else {
+#pragma unroll
+                    for (int q = 0; q < kU; q += kRowsDma) dma_filler(sh, a.tab, lane16);
                 }
             }
             // the addresses of the block's LDS accesses: ring slots of the
-            // reads (the last kDin steps may wrap to the ring's start), table
-            // slots, DMA targets and sources
-            const T *pin = &in_ring[t0 % kZ][r][0];
-            const T *pin_hi = (t0 % kZ == kZ - kU) ? pin - kZ * kRows * kCols : pin;
-            const int sb = t0 % kD;
-            const Pair<T> *psc = &sh.scr[g][sb][lane_entry(i)];
-            const Pair<T> *psc_hi = (sb == kD - kU) ? psc - kD * kLanes * S : psc;
-            const unsigned m0b = lds_addr(&sh.scr[g][0][0]) + (unsigned)sb * kStepBytes;
-            const char *srcb = tab_band + (long long)(t0 + kD) * kStepBytes;  // step t0+kD+K: the DMA of step u, K = u+1-kSPD
-            // step u's output (the row-end values of the last sequence, lane
-            // 15 of each row) is broadcast along its row and kept by lane u;
-            // the block's kU outputs are stored together after its last step
-            T outv[kCols];
-#pragma unroll
-            for (int c = 0; c < kCols; ++c) outv[c] = T(0);
+            // reads (the last kDin steps read the next block's), table slots,
+            // DMA targets
+            const unsigned tab0 = kD == kU ? 0u : (unsigned)(t0 % kD) * kStepBytes;
+            const unsigned tab1 = kD == kU ? 0u : (unsigned)((t0 + kU) % kD) * kStepBytes;
+            set_m0(m0_base + tab0);
+            const char *src = tab_band + (long long)(t0 + kD) * kStepBytes;  // step t0+kD+K: the DMA of step u, K = u+1-kSPD
+            const unsigned pin_next = in_lane + ((unsigned)(t0 + kU) % kZ) * kSlotBytes;
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
                 // keep each step's instructions together: the entries and
-                // rows read for the next steps then have a whole step of
+                // rows read for the steps after next then have two steps of
                 // issue time to arrive before their first use
+                __builtin_amdgcn_sched_barrier(0);
+                const Pair<T> in = inbuf[u % kDin];
+                inbuf[u % kDin] = u + kDin >= kU ? lds_at<Pair<T>>(pin_next)[(u + kDin - kU) * kRows]
+                                                 : lds_at<Pair<T>>(pin)[(u + kDin) * kRows];
+                const SC<MC> sc = scn[u % kAhead];
+                if ((u + kAhead) % kSPD == 0) {
+                    // from the second DMA of the block on, its own are the youngest
+                    if (u < kU - kSPD) wait_block<kExtra>();
+                    else wait_block();
+                }
+                read_sc((u + kAhead) % kU, scn[u % kAhead], u + kAhead < kU ? tab0 : tab1);
+                // the reads above are issued before the step's arithmetic
                 __builtin_amdgcn_sched_barrier(0);
                 T X0[kCols];
 #pragma unroll
-                for (int c = 0; c < kCols; ++c) X0[c] = shift_in(inbuf[u % kDin][c], E[S - 1][c]);
-                {
-                    const T *q = (u + kDin >= kU ? pin_hi : pin) + (u + kDin) * kRows * kCols;
+                for (int c = 0; c < kCols; ++c) X0[c] = shift_in(c == 0 ? in.x : in.y, E[S - 1][c]);
+                // the last sequence's outputs of the step before
 #pragma unroll
-                    for (int c = 0; c < kCols; ++c) inbuf[u % kDin][c] = lds_ld(q + c);
+                for (int c = 0; c < kCols; ++c) {
+                    T &k = outv[u >> 2][c];
+                    switch (u & 3) {  // a constant once the loop is unrolled
+                        case 0: k = row_end<0>(k, E[S - 1][c]); break;
+                        case 1: k = row_end<1>(k, E[S - 1][c]); break;
+                        case 2: k = row_end<2>(k, E[S - 1][c]); break;
+                        default: k = row_end<3>(k, E[S - 1][c]); break;
+                    }
                 }
-                const SC sc = scn;
-                if ((u + 1) % kSPD == 0) wait_block();
-                {
-                    const Pair<T> *q = (u + 1 >= kU ? psc_hi : psc) + (u + 1) * kLanes * S;
-#pragma unroll
-                    for (int s2 = 0; s2 < S; ++s2) scn.p[s2] = q[s2 * kSlotStride];
-                }
-                // the reads above are issued before this step's arithmetic
-                __builtin_amdgcn_sched_barrier(0);
-                rotate<MASK>(Y, E, X0, sc, m, m1);
+                carry(Y, ap);
+                emit(Y, E, X0, sc, ap);
                 if (u % kSPD == kSPD - 1) {
                     // u is a constant once the loop is unrolled
                     switch (u + 1 - kSPD) {
-                        case 0: dma_block_at<0>(m0b, srcb, lane16, E[0][0]); break;
-                        case 2: dma_block_at<2>(m0b, srcb, lane16, E[0][0]); break;
-                        case 4: dma_block_at<4>(m0b, srcb, lane16, E[0][0]); break;
-                        case 6: dma_block_at<6>(m0b, srcb, lane16, E[0][0]); break;
+                        case 0: dma_block_at<0>(src, lane16, E[S - 1][0]); break;
+                        case 2: dma_block_at<2>(src, lane16, E[S - 1][0]); break;
+                        case 4: dma_block_at<4>(src, lane16, E[S - 1][0]); break;
+                        case 6: dma_block_at<6>(src, lane16, E[S - 1][0]); break;
                         default: break;
                     }
                 }
-#pragma unroll
-                for (int c = 0; c < kCols; ++c) {
-                    const T b = row_end(E[S - 1][c]);
-                    outv[c] = i == u ? b : outv[c];
-                }
             }
+            pin = pin_next;
             // a split part's last band publishes the rows the previous block
             // stored: they are complete once at most this block's DMAs are
             // outstanding (vector memory operations complete in issue order)
-            if (split_out >= 0 && pub > published) {
+            if (LINK && split_out >= 0 && pub > published) {
                 asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kU / kSPD) : "memory");
                 if (lane == 0) __hip_atomic_store(a.prog + split_out, pub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 published = pub;
             }
-            // lane i < kU of each row stores output position po0 + i: to the
-            // next band's ring up to ring_hi, else (leaving the chain or the
-            // part) to its row of A; positions outside [0, R] carry no row.
-            // (The global stores only lengthen the table waits that follow
-            // them: those wait for the DMAs issued before them, and loads
-            // return in order.)
-            {
-                const int po = po0 + i;
-                if (i < kU && po >= 0 && po <= R) {
-                    if (po <= ring_hi) {
-                        T *dst = &out_ring[(po + npa_next) % kZ][r][0];
-#pragma unroll
-                        for (int c = 0; c < kCols; ++c) lds_st(dst + c, outv[c]);
-                    } else if (split_out >= 0) {
-#pragma unroll
-                        for (int c = 0; c < kCols; ++c)
-                            if (colv[c] >= 0)
-                                __hip_atomic_store(aptr(c, row_of(po)), outv[c], __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-                    } else {
-#pragma unroll
-                        for (int c = 0; c < kCols; ++c)
-                            if (colv[c] >= 0) *aptr(c, row_of(po)) = outv[c];
-                    }
+            // the block's outputs, positions po0 .. po0+kU-1: to the next
+            // band's ring up to ring_hi, else (leaving the chain or the part)
+            // to their rows of A; positions outside [0, R] carry no row
+            const T ve = (i & 1) ? outv[1][0] : outv[0][0];
+            const T vo = (i & 1) ? outv[1][1] : outv[0][1];
+            const T v = out_c ? vo : ve;
+            if (!LINK && (unsigned)(t0 - t_same) < (unsigned)n_same) {
+                if (END & kLast && last) {
+                    if (out_on) *out_a = v;
+                } else {
+                    *lds_at<T>(out_lane + ((unsigned)t0 + out_slot0) % kZ * kSlotBytes) = v;
+                    pub_avail = out_base + (t0 + kU - kLag - off) + out_off;
+                    if (END & kLast) dma_filler(sh, a.tab, lane16);
                 }
+            } else {
+                const int po0 = t0 - kLag - off, po = po0 + out_u;
+                if (po0 + kU > 0) {
+                    if (po >= 0 && po <= R) {
+                        if (po <= ring_hi) {
+                            out_ring[(((po + out_off) & (kZ - 1)) * kRows + r) * kCols + out_c] = v;
+                        } else if (out_on) {
+                            if (split_out >= 0) __hip_atomic_store(out_a, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                            else *out_a = v;
+                        }
+                    }
+                    if (ring_hi >= 0) pub_avail = max(pub_avail, out_base + min(po0 + kU - 1, ring_hi) + out_off + 1);
+                    pub = max(0, min(po0 + kU, R + 1));
+                }
+                // unless some lane stored a row of A
+                if (END & kLast && max(max(po0, ring_hi + 1), 0) > min(po0 + kU - 1, R)) dma_filler(sh, a.tab, lane16);
             }
-            pub = max(0, min(po0 + kU, R + 1));
-            if (!ok) break;
-            // publish what the block wrote and read
-            __atomic_signal_fence(__ATOMIC_SEQ_CST);
-            if (!last && lane == 0) lds_st(&sh.avail[g + 1], written);
-            // positions read, never beyond this chain's part of the ring
-            if (lane == 0) lds_st(&sh.freed[g], in_base + min(t0 + kU, span(R)));
+            out_a += astep * kU;
+            t0 += kU;
+            // publish what the block read (never beyond this chain's part of
+            // the ring) and wrote
+            pub_freed = min(in_base + t0, in_free_end);
+            asm volatile("s_mov_b64 exec, 1\n\tds_write2_b32 %0, %1, %2 offset1:1\n\ts_mov_b64 exec, -1"
+                         :
+                         : "v"(pub_lds), "v"(pub_freed), "v"(pub_avail)
+                         : "memory");
         }
 
-        if (!ok) {
-            fail(sh);
-            atomicOr(a.ctl + FTAMD_SYS_CTL_ERR, FTAMD_ERR_TIMEOUT);
-            return false;
-        }
-        if (split_out >= 0) {
+        if (LINK && split_out >= 0) {
             // every row stored and complete
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             if (lane == 0) __hip_atomic_store(a.prog + split_out, R + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-#ifdef FTAMD_TRACE
-        if (a.trace && lane == 0) {
-            // accumulated over the bands the wave runs
-            unsigned long long *rec = a.trace + ((long long)blockIdx.x * kWaves + g) * 8;
-            if (rec[0] == 0) rec[0] = tr_start;
-            rec[1] = wall_clock64();
-            rec[2] += __builtin_amdgcn_s_memtime() - tr_c0;
-            rec[3] += tr_in();
-            rec[4] += tr_out();
-            rec[5] += steps;
-            rec[6] += R;
-            rec[7] += tr_dma();
-        }
-#endif
         return true;
     }
 
-    // Ring positions one band's stream takes: its R + 1 positions rounded up
-    // to whole rings, so that every stream starts at ring slot 0.
-    __device__ static int span(int R) { return (R + kZ) / kZ * kZ; }
+    // Ring slots one band's stream takes: its R + 1 positions from slot `off`
+    // on, rounded up to whole rings, so that every stream starts at ring slot 0.
+    __device__ static int span(int R, int off) { return (R + off + kZ) / kZ * kZ; }
+
+    // Idle steps (and ring slots) before position 0 of the stream of a part's
+    // band w.  A block needs input up to kDin slots past its own; with kDin
+    // more idle steps than the band before, that is where a block of the band
+    // before ends, and it follows that band by kLag + kU + kDin steps (without,
+    // by up to kU - kDin more).
+    __device__ static int idle(int w) { return (kDin * w) & (kU - 1); }
 
     // XCD (accelerator complex die, with its own L2) this workgroup runs on.
     __device__ static int xcd_id(int nxcd) {
@@ -626,12 +726,11 @@ struct Engine {
     // however many workgroups the hardware runs at once.
     __device__ static void run(const FtamdSysLaunch &a, Shared &sh) {
         {
-            T *rp = &sh.ring[0][0][0][0];
+            T *rp = (T *)&sh.ring[0][0][0];
             for (int x = threadIdx.x; x < kWaves * kZ * kRows * kCols; x += blockDim.x) rp[x] = T(0);
-            if (threadIdx.x < kWaves) {
-                sh.avail[threadIdx.x] = 0;
-                sh.freed[threadIdx.x] = 0;
-            }
+            Pair<T> *id = &sh.ident[0][0];
+            for (int x = threadIdx.x; x < kD * kLanes * S; x += blockDim.x) id[x] = Pair<T>{T(0), T(1)};
+            if (threadIdx.x < kWaves + 2) sh.pub[threadIdx.x].freed = sh.pub[threadIdx.x].avail = 0;
             if (threadIdx.x == 0) sh.abort_flag = 0;
         }
         const int lane = threadIdx.x & 63;
@@ -647,12 +746,17 @@ struct Engine {
             const int t = uniform(lds_ld(&sh.slot));
             if (t >= ns || uniform(lds_ld(&sh.abort_flag))) break;
             const int slot = s0 + t;
-            const int it0 = uniform(a.slot_items[slot]), it1 = uniform(a.slot_items[slot + 1]);
+            const ConstInt *slot_items = (const ConstInt *)(uintptr_t)a.slot_items;
+            const int it0 = slot_items[slot], it1 = slot_items[slot + 1];
             for (int it = it0; it < it1; ++it) {
-                const FtamdSysChain &ch = a.chains[uniform(a.items[it].chain)];
+                const ConstItem &item = ((const ConstItem *)(uintptr_t)a.items)[it];
+                const int chain = uniform(item.chain);
+                const ConstChain &ch = ((const ConstChain *)(uintptr_t)a.chains)[chain];
                 const int nb = uniform(ch.nb), b0 = uniform(ch.band0);
-                const int w = g - uniform(a.items[it].wave0);  // this wave's band of the part, if any
-                if (w >= 0 && w < nb) {
+                const int w = g - uniform(item.wave0);  // this wave's band of the part, if any
+                if (w < -1 || w >= nb) continue;
+                const ConstBand *bands = (const ConstBand *)(uintptr_t)a.bands + b0;
+                if (w >= 0) {
                     switch (uniform(ch.prio)) {
                         case 3: __builtin_amdgcn_s_setprio(3); break;
                         case 2: __builtin_amdgcn_s_setprio(2); break;
@@ -664,24 +768,35 @@ struct Engine {
                     // per lane row serves both columns (sph and disk: the two
                     // columns of a row are the cosine and sine columns of one
                     // order, so they apply the same sequences)
-                    const int gbase = uniform(a.bands[b0 + w].gbase);
-                    const int glast = gbase + uniform(a.bands[b0 + w].nseq) - 1;
+                    const int gbase = uniform(bands[w].gbase);
+                    const int glast = gbase + uniform(bands[w].nseq) - 1;
                     bool masked = false;
+#pragma unroll
                     for (int k = 0; k < FTAMD_SYS_COLS; ++k)
                         masked |= ch.col[k] >= 0 && (ch.glo[k] > gbase || ch.ghi[k] < glast);
-                    // bands that hand rows to or take rows from another
-                    // part of the chain run their own instantiation, so the
-                    // others carry none of that code
+                    // the kinds of bands run their own instantiations, so
+                    // that each carries only its own code
                     const bool link = (w == 0 && uniform(ch.split_in) >= 0) || (w == nb - 1 && uniform(ch.split_out) >= 0);
                     constexpr int MK = ROWMASK ? 1 : 2;
-                    const bool ok = link ? (!masked ? run_band<0, true>(a, sh, ch, w, g, lane, in_base, out_base)
-                                                    : run_band<MK, true>(a, sh, ch, w, g, lane, in_base, out_base))
-                                         : (!masked ? run_band<0, false>(a, sh, ch, w, g, lane, in_base, out_base)
-                                                    : run_band<MK, false>(a, sh, ch, w, g, lane, in_base, out_base));
+                    const FtamdSysChain &cv = a.chains[chain];
+                    const bool f = w == 0, l = w == nb - 1;
+                    bool ok;
+#define FTAMD_RUN_BAND(mask, end, lk) run_band<mask, end, lk>(a, sh, ch, cv, w, g, lane, in_base, out_base)
+                    if (link) ok = FTAMD_RUN_BAND(MK, kBoth, true);
+                    else if (masked && f && !l) ok = FTAMD_RUN_BAND(MK, kFirst, false);
+                    else if (masked && l && !f) ok = FTAMD_RUN_BAND(MK, kLast, false);
+                    else if (masked) ok = FTAMD_RUN_BAND(MK, kBoth, false);
+                    else if (f) ok = l ? FTAMD_RUN_BAND(0, kBoth, false) : FTAMD_RUN_BAND(0, kFirst, false);
+                    else ok = l ? FTAMD_RUN_BAND(0, kLast, false) : FTAMD_RUN_BAND(0, kInner, false);
+#undef FTAMD_RUN_BAND
                     if (!ok) break;
-                    in_base += span(uniform(a.bands[b0 + w].R));
+                    const int R = uniform(bands[w].R);
+                    in_base += span(R, idle(w));
                 }
-                if (w + 1 >= 0 && w + 1 < nb) out_base += span(uniform(a.bands[b0 + w + 1].R));
+                if (w + 1 < nb) {
+                    const int R = uniform(bands[w + 1].R);
+                    out_base += span(R, idle(w + 1));
+                }
             }
             __builtin_amdgcn_s_setprio(0);
             __syncthreads();
