@@ -5,23 +5,27 @@
 // along phi (c2r / r2c), with the reference's scalings and the column layout
 // of its data_r2c / data_c2r (fftw.c:40-60).
 //
-// The DCTs run as complex FFTs of length N (hipFFT; the synthesis plans put
-// two columns in one FFT) between two HIP kernels, by Makhoul's reordering: DCT-II(x)_k = 2 Re(e^{-i pi k/2N} FFT(v)_k) with
-// v_m = x_{2m}, v_{N-1-m} = x_{2m+1}; DCT-III(X) is the inverse map,
-// v = IFFT(e^{i pi k/2N} (X_k - i X_{N-k})) (unnormalized, X_N = 0),
-// y_{2m} = Re v_m, y_{2m+1} = Re v_{N-1-m}.  The DSTs are DCTs of the
-// reversed input with alternating output signs (DST-III) or of the
-// sign-alternated input with reversed output (DST-II).  The phi DFTs are
-// hipFFT's strided transforms (row i is the transform at element i, stride
-// N); with N even, rows 2p and 2p+1 share one complex DFT over X read as
-// N/2 x M complex.
+// The DCTs run as complex FFTs of length N by Makhoul's reordering:
+// DCT-II(x)_k = 2 Re(e^{-i pi k/2N} FFT(v)_k) with v_m = x_{2m}, v_{N-1-m} =
+// x_{2m+1}; DCT-III(X) is the inverse map, v = IFFT(e^{i pi k/2N} (X_k - i
+// X_{N-k})) (unnormalized, X_N = 0), y_{2m} = Re v_m, y_{2m+1} = Re v_{N-1-m}.
+// The DSTs are DCTs of the reversed input with alternating output signs
+// (DST-III) or of the sign-alternated input with reversed output (DST-II).
+//
+// The sphere's, the vector field's, the annulus's and the disk's grids take
+// two launches of the line transforms (ft_dft.hpp).  Lengths those do not
+// take (above FTAMD_DFT_MAX), the disk's DCT-IV and the other geometries run
+// hipFFT between kernels: there the synthesis plans put two columns in one
+// FFT, and the phi DFTs are hipFFT's strided transforms (row i is the
+// transform at element i, stride N); with N even, rows 2p and 2p+1 share one
+// complex DFT over X read as N/2 x M complex.
 #include <hip/hip_runtime.h>
 #include <hipfft/hipfft.h>
 
 #include <math.h>
 #include <stdlib.h>
 
-#include "ft_hip_abi.h"
+#include "ft_lines.hpp"
 
 struct FtamdGrid {
     int N, M, type3;
@@ -30,13 +34,14 @@ struct FtamdGrid {
     int nsin;     // sine-class columns (disk)
     int pair;     // phi DFTs of two real rows as one complex DFT (N even)
     int tpair;    // theta FFTs of two columns as one (synthesis, not the disk): column j in part j & 1 of line j / 2
+    FtamdDft *dft_theta, *dft_phi;  // the line transforms, both or neither (lengths they take): then no theta, phi, Z, Yp
     hipfftHandle theta, phi, iv;
     hipfftHandle phi_r;  // the real phi DFTs of a paired plan, made on first use (X not 16-byte aligned)
     double2 *tw;  // e^{i pi k / 2N}, k < N
     double2 *tw4; // e^{i pi (2k+1) / 4N}, k < N (disk)
     double2 *Z;   // N x M complex: the columns' FFTs
     double2 *Z4;  // 2N x nsin complex: the disk's sine-class columns, zero-padded (disk)
-    double2 *Y;   // N x (M/2+1) complex: the rows' half spectra (paired, not the disk: N/2 x M full spectra)
+    double2 *Y;   // N x (M/2+1) complex: the rows' half spectra (hipFFT, paired, not the disk: N/2 x M full spectra)
     double2 *Yp;  // the disk's paired plans: N/2 x M full spectra of the row pairs
     double *w;    // the annulus's radial weights (N), NULL otherwise
 };
@@ -473,9 +478,14 @@ extern "C" int ftamd_grid_create(int N, int M, int type3, int plan_mode, const d
         tw[k] = make_double2((double)cosl(th), (double)sinl(th));
     }
     if (rc == FTAMD_OK && hipMalloc((void **)&g->tw, sizeof(double2) * (size_t)N) != hipSuccess) rc = FTAMD_ENOMEM;
-    if (rc == FTAMD_OK && hipMalloc((void **)&g->Z, zbytes) != hipSuccess) rc = FTAMD_ENOMEM;
+    const bool lines = ftamd_dft_fits(N) && ftamd_dft_fits(M);
+    if (lines) {
+        if (rc == FTAMD_OK) rc = ftamd_dft_create(N, &g->dft_theta);
+        if (rc == FTAMD_OK) rc = ftamd_dft_create(M, &g->dft_phi);
+    }
+    if (rc == FTAMD_OK && !lines && hipMalloc((void **)&g->Z, zbytes) != hipSuccess) rc = FTAMD_ENOMEM;
     if (rc == FTAMD_OK && hipMalloc((void **)&g->Y, ybytes) != hipSuccess) rc = FTAMD_ENOMEM;
-    if (rc == FTAMD_OK && g->pair && g->disk &&
+    if (rc == FTAMD_OK && !lines && g->pair && g->disk &&
         hipMalloc((void **)&g->Yp, sizeof(double2) * (size_t)(N / 2) * M) != hipSuccess)
         rc = FTAMD_ENOMEM;
     if (rc == FTAMD_OK && hipMemcpy(g->tw, tw, sizeof(double2) * (size_t)N, hipMemcpyHostToDevice) != hipSuccess)
@@ -502,14 +512,14 @@ extern "C" int ftamd_grid_create(int N, int M, int type3, int plan_mode, const d
         else if (hipMemcpy(g->w, w, sizeof(double) * (size_t)N, hipMemcpyHostToDevice) != hipSuccess) rc = FTAMD_EDEVICE;
     }
     /* the sine-class slots of Z stay zero in the disk's plans (never written) */
-    if (rc == FTAMD_OK && g->disk && hipMemset(g->Z, 0, zbytes) != hipSuccess) rc = FTAMD_EDEVICE;
+    if (rc == FTAMD_OK && !lines && g->disk && hipMemset(g->Z, 0, zbytes) != hipSuccess) rc = FTAMD_EDEVICE;
     // theta: M contiguous complex transforms of length N
     int n1[1] = {N};
-    if (rc == FTAMD_OK)
+    if (rc == FTAMD_OK && !lines)
         rc = fft_ok(hipfftPlanMany(&g->theta, 1, n1, n1, 1, N, n1, 1, N, HIPFFT_Z2Z, g->tpair ? (M + 1) / 2 : M));
     // phi: N real transforms of length M, element i of row-transform e at e + i*N; paired, N/2
     // complex ones, element i of pair p at p + i*N/2
-    if (rc == FTAMD_OK) rc = g->pair ? phi_plan_pair(g) : phi_plan_real(g, &g->phi);
+    if (rc == FTAMD_OK && !lines) rc = g->pair ? phi_plan_pair(g) : phi_plan_real(g, &g->phi);
     if (rc != FTAMD_OK) {
         ftamd_grid_destroy(g);
         return rc;
@@ -521,6 +531,8 @@ extern "C" int ftamd_grid_create(int N, int M, int type3, int plan_mode, const d
 extern "C" void ftamd_grid_destroy(FtamdGrid *g) {
     if (!g) return;
     hipDeviceSynchronize();
+    ftamd_dft_destroy(g->dft_theta);
+    ftamd_dft_destroy(g->dft_phi);
     if (g->theta) hipfftDestroy(g->theta);
     if (g->phi) hipfftDestroy(g->phi);
     if (g->phi_r) hipfftDestroy(g->phi_r);
@@ -541,19 +553,8 @@ extern "C" int ftamd_grid_run(FtamdGrid *g, double *X, int exec_sphv, double f0,
     const int N = g->N, M = g->M;
     const hipStream_t st = (hipStream_t)stream;
     const dim3 block(256), grid((N + 255) / 256, M);
-    // the paired phi DFTs read or write X as complex: 16-byte aligned X only, else the real DFTs
-    const int pair = g->pair && ((uintptr_t)X & 15) == 0;
-    if (g->pair && !pair && !g->phi_r) {
-        const int r = phi_plan_real(g, &g->phi_r);
-        if (r != FTAMD_OK) return r;
-    }
-    const hipfftHandle phi = g->pair && !pair ? g->phi_r : g->phi;
-    const dim3 gridp((N / 2 + 255) / 256, M / 2 + 1);
-    const int tp = g->tpair;
-    int rc = fft_ok(hipfftSetStream(g->theta, st));
-    if (rc == FTAMD_OK) rc = fft_ok(hipfftSetStream(phi, st));
-    if (rc == FTAMD_OK && g->iv) rc = fft_ok(hipfftSetStream(g->iv, st));
-    if (rc != FTAMD_OK) return rc;
+    int rc = FTAMD_OK;
+    if (g->iv && (rc = fft_ok(hipfftSetStream(g->iv, st))) != FTAMD_OK) return rc;
     const int iv = g->disk && g->nsin > 0;
     const dim3 grid4((2 * N + 255) / 256, g->nsin > 0 ? g->nsin : 1), grid4o((N + 255) / 256, g->nsin > 0 ? g->nsin : 1);
     // the disk's sine class: DCT-IV of the columns (synthesis plans, before the phi DFT)
@@ -574,6 +575,39 @@ extern "C" int ftamd_grid_run(FtamdGrid *g, double *X, int exec_sphv, double f0,
         hipLaunchKernelGGL(ftgrid::post4_x, grid4o, block, 0, st, g->Z4, X, g->tw4, N, g->nsin, f1);
         return hipGetLastError() == hipSuccess ? FTAMD_OK : FTAMD_EDEVICE;
     };
+    // Lengths the line transforms take: two launches (and the disk's DCT-IV
+    // between them).  Synthesis / analysis at n = 1024 (1024 x 2047): 47 / 52 us,
+    // against 99 / 104 us of the path below (hipFFT between kernels that
+    // reorder and scale); N = 451, M = 901: 24 against 59 us.
+    if (g->dft_theta) {
+        FtamdLines l = {X, g->Y, g->tw, g->w, 0, 0, N, M, g->plan_sphv, exec_sphv, iv, g->w ? wmode : 0,
+                        N % 2 == 0 && ((uintptr_t)X & 15) == 0, f0, f1, a, b, 0, NULL, NULL, NULL};
+        auto pass = [&](const FtamdDft *d, int kind) {
+            l.kind = kind;
+            l.lines = kind <= FTAMD_LINES_THETA2 ? M / 2 + 1 : (N + 1) / 2;
+            return ftamd_dft_lines(d, &l, stream);
+        };
+        if (g->type3) {
+            rc = pass(g->dft_theta, FTAMD_LINES_THETA3);
+            if (rc == FTAMD_OK && iv) rc = iv_from_x();
+            return rc == FTAMD_OK ? pass(g->dft_phi, FTAMD_LINES_PHI_BACK) : rc;
+        }
+        rc = pass(g->dft_phi, FTAMD_LINES_PHI_FWD);
+        if (rc == FTAMD_OK && iv) rc = iv_from_y();
+        return rc == FTAMD_OK ? pass(g->dft_theta, FTAMD_LINES_THETA2) : rc;
+    }
+    // the paired phi DFTs read or write X as complex: 16-byte aligned X only, else the real DFTs
+    const int pair = g->pair && ((uintptr_t)X & 15) == 0;
+    if (g->pair && !pair && !g->phi_r) {
+        const int r = phi_plan_real(g, &g->phi_r);
+        if (r != FTAMD_OK) return r;
+    }
+    const hipfftHandle phi = g->pair && !pair ? g->phi_r : g->phi;
+    const dim3 gridp((N / 2 + 255) / 256, M / 2 + 1);
+    const int tp = g->tpair;
+    rc = fft_ok(hipfftSetStream(g->theta, st));
+    if (rc == FTAMD_OK) rc = fft_ok(hipfftSetStream(phi, st));
+    if (rc != FTAMD_OK) return rc;
     if (g->type3) {
         // fix-ups f0 (row 0, cosine columns) and f1 (last row, sine columns),
         // DCT-III / DST-III (the disk: DCT-IV on the sine class), scalings,
