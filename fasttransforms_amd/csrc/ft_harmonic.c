@@ -343,54 +343,54 @@ static int valid(int transform, char TRANS, const ft_harmonic_plan *P, int N, in
     return P->RP[0]->kind == geo && P->NP >= np && N == P->RP[0]->n && M >= 1 && ftamd_valid_M(rk, N, M);
 }
 
-/* One product into the work buffer and back into dA. */
-static int product(struct ftamd_harmonic_dev *d, FtamdTrmmLaunch *t, void *dA, size_t bytes, void *stream) {
-    t->X = dA;
-    t->Y = d->dY;
-    int rc = ftamd_hip_trmm_launch(t, stream);
-    if (rc == FTAMD_OK) rc = ftamd_hip_d2d(dA, d->dY, bytes, stream);
-    return rc;
+/* The products p[0 .. np-1] (one or two), one after another, on dA: the
+ * first into the work buffer, a second from there back into dA. */
+static int products(struct ftamd_harmonic_dev *d, FtamdTrmmLaunch *p, int np, void *dA, size_t bytes, void *stream) {
+    p[0].X = dA;
+    p[0].Y = d->dY;
+    int rc = ftamd_hip_trmm_launch(&p[0], stream);
+    if (rc != FTAMD_OK) return rc;
+    if (np == 1) return ftamd_hip_d2d(dA, d->dY, bytes, stream);
+    p[1].X = d->dY;
+    p[1].Y = dA;
+    return ftamd_hip_trmm_launch(&p[1], stream);
+}
+
+/* The product on the column classes j = c mod ncls from the left. */
+static FtamdTrmmLaunch class_product(int ncls, int trans, int n, int M) {
+    FtamdTrmmLaunch t;
+    memset(&t, 0, sizeof(t));
+    t.n = n;
+    t.M = M;
+    t.cstride = ncls;
+    t.ncls = ncls;
+    t.trans = trans;
+    return t;
+}
+
+/* One triangle product on every column (left) or every row (right). */
+static FtamdTrmmLaunch tri_product(const double *U, int right, int trans, int n, int M) {
+    FtamdTrmmLaunch t = class_product(1, trans, n, M);
+    t.U[0] = U;
+    t.right = right;
+    return t;
 }
 
 /* The products of the column-class transforms (sph, sphv, disk). */
 static int class_products(struct ftamd_harmonic_dev *d, double *const *H, int vec, int trans, int n, int M, void *dA,
                           size_t bytes, void *stream) {
-    FtamdTrmmLaunch t;
-    memset(&t, 0, sizeof(t));
+    FtamdTrmmLaunch t = class_product(4, trans, n, M);
     for (int c = 0; c < 4; c++) {
         const int even = (c == 0 || c == 3); /* columns of even-parity orders (sph and disk layouts) */
         t.U[c] = H[even != vec ? 0 : 1];
-        const int count = M > c ? (M - c + 3) / 4 : 0;
-        t.ctiles[c] = (count + FTAMD_TRMM_COLS - 1) / FTAMD_TRMM_COLS;
     }
-    t.n = n;
-    t.M = M;
-    t.cstride = 4;
-    t.ncls = 4;
-    t.trans = trans;
-    return product(d, &t, dA, bytes, stream);
-}
-
-/* One triangle product on every column (left) or every row (right). */
-static int tri_product(struct ftamd_harmonic_dev *d, const double *U, int right, int trans, int n, int M, void *dA,
-                       size_t bytes, void *stream) {
-    FtamdTrmmLaunch t;
-    memset(&t, 0, sizeof(t));
-    t.U[0] = U;
-    t.ctiles[0] = (M + FTAMD_TRMM_COLS - 1) / FTAMD_TRMM_COLS;
-    t.n = n;
-    t.M = M;
-    t.cstride = 1;
-    t.ncls = 1;
-    t.trans = trans;
-    t.right = right;
-    return product(d, &t, dA, bytes, stream);
+    return products(d, &t, 1, dA, bytes, stream);
 }
 
 /* The triangle's transforms (drivers.c:921-957): tri2cheb 'N' is hi2lo, P[0]
  * from the left unless (alpha, beta + gamma) = (-1/2, -3/2), P[1]^T from the
  * right unless beta = gamma = -1/2, then the Chebyshev normalization;
- * cheb2tri inverts it. */
+ * cheb2tri inverts it.  The normalization goes with the product beside it. */
 static int run_tri(ft_harmonic_plan *P, int inverse, char TRANS, void *dA, int M, size_t bytes, void *stream) {
     struct ftamd_harmonic_dev *d = P->dev;
     const int n = P->RP[0]->n;
@@ -399,28 +399,26 @@ static int run_tri(ft_harmonic_plan *P, int inverse, char TRANS, void *dA, int M
     const double s1 = inverse ? 1.41421356237309504880 : 0.70710678118654752440; /* M_SQRT2, M_SQRT1_2 */
     const double s2 = inverse ? 1.57079632679489661923 : 0.63661977236758134308; /* M_PI_2, M_2_PI */
     double *const *H = inverse ? d->dPinv : d->dP;
-    int rc = FTAMD_OK;
-    if (!inverse && TRANS == 'N') {
-        rc = ft_gpu_execute(P->RP[0], FT_GPU_TRI, 0, FT_GPU_FP64, dA, M, stream);
-        if (rc == FTAMD_OK && use0) rc = tri_product(d, H[0], 0, 0, n, M, dA, bytes, stream);
-        if (rc == FTAMD_OK && use1) rc = tri_product(d, H[1], 1, 1, n, M, dA, bytes, stream);
-        if (rc == FTAMD_OK) rc = ftamd_hip_cheb_scale(dA, n, M, s1, s2, stream);
-    } else if (!inverse) {
-        rc = ftamd_hip_cheb_scale(dA, n, M, s1, s2, stream);
-        if (rc == FTAMD_OK && use1) rc = tri_product(d, H[1], 1, 0, n, M, dA, bytes, stream);
-        if (rc == FTAMD_OK && use0) rc = tri_product(d, H[0], 0, 1, n, M, dA, bytes, stream);
-        if (rc == FTAMD_OK) rc = ft_gpu_execute(P->RP[0], FT_GPU_TRI, 1, FT_GPU_FP64, dA, M, stream);
-    } else if (TRANS == 'N') {
-        rc = ftamd_hip_cheb_scale(dA, n, M, s1, s2, stream);
-        if (rc == FTAMD_OK && use1) rc = tri_product(d, H[1], 1, 1, n, M, dA, bytes, stream);
-        if (rc == FTAMD_OK && use0) rc = tri_product(d, H[0], 0, 0, n, M, dA, bytes, stream);
-        if (rc == FTAMD_OK) rc = ft_gpu_execute(P->RP[0], FT_GPU_TRI, 1, FT_GPU_FP64, dA, M, stream);
-    } else {
-        rc = ft_gpu_execute(P->RP[0], FT_GPU_TRI, 0, FT_GPU_FP64, dA, M, stream);
-        if (rc == FTAMD_OK && use0) rc = tri_product(d, H[0], 0, 1, n, M, dA, bytes, stream);
-        if (rc == FTAMD_OK && use1) rc = tri_product(d, H[1], 1, 0, n, M, dA, bytes, stream);
-        if (rc == FTAMD_OK) rc = ftamd_hip_cheb_scale(dA, n, M, s1, s2, stream);
+    const int trans = TRANS == 'T';
+    const int fwd = inverse ? trans : !trans; /* rotations before the products */
+    FtamdTrmmLaunch p[2];
+    int np = 0, rc = FTAMD_OK;
+    if (!fwd && use1) p[np++] = tri_product(H[1], 1, !trans, n, M);
+    if (use0) p[np++] = tri_product(H[0], 0, trans, n, M);
+    if (fwd && use1) p[np++] = tri_product(H[1], 1, !trans, n, M);
+    if (np && fwd) {
+        p[np - 1].scale_out = 1;
+        p[np - 1].post1 = s1;
+        p[np - 1].post2 = s2;
+    } else if (np) {
+        p[0].scale_in = 1;
+        p[0].pre1 = s1;
+        p[0].pre2 = s2;
     }
+    if (fwd) rc = ft_gpu_execute(P->RP[0], FT_GPU_TRI, 0, FT_GPU_FP64, dA, M, stream);
+    if (rc == FTAMD_OK)
+        rc = np ? products(d, p, np, dA, bytes, stream) : ftamd_hip_cheb_scale(dA, n, M, s1, s2, stream);
+    if (rc == FTAMD_OK && !fwd) rc = ft_gpu_execute(P->RP[0], FT_GPU_TRI, 1, FT_GPU_FP64, dA, M, stream);
     return rc;
 }
 
@@ -430,42 +428,19 @@ static int run_tri(ft_harmonic_plan *P, int inverse, char TRANS, void *dA, int M
  * cheb2rectdisk inverts it with Pinv in reverse order. */
 static int run_rectdisk(ft_harmonic_plan *P, int inverse, char TRANS, void *dA, int M, size_t bytes, void *stream) {
     struct ftamd_harmonic_dev *d = P->dev;
-    const int n = P->RP[0]->n;
+    const int n = P->RP[0]->n, trans = TRANS == 'T';
     double *const *H = inverse ? d->dPinv : d->dP;
-    FtamdTrmmLaunch t;
-    memset(&t, 0, sizeof(t));
-    t.n = n;
-    t.M = M;
-    t.cstride = 2;
-    t.ncls = 2;
-    for (int c = 0; c < 2; c++) {
-        t.U[c] = H[c];
-        const int count = M > c ? (M - c + 1) / 2 : 0;
-        t.ctiles[c] = (count + FTAMD_TRMM_COLS - 1) / FTAMD_TRMM_COLS;
-    }
-    const int fwd = !inverse ? TRANS == 'N' : TRANS == 'T'; /* rotations before the products */
+    const int fwd = inverse ? trans : !trans; /* rotations before the products */
+    FtamdTrmmLaunch p[2];
+    FtamdTrmmLaunch *left = &p[fwd ? 0 : 1];
+    *left = class_product(2, trans, n, M);
+    left->U[0] = H[0];
+    left->U[1] = H[1];
+    p[fwd ? 1 : 0] = tri_product(H[2], 1, !trans, n, M);
     int rc = FTAMD_OK;
-    if (fwd && !inverse) {
-        rc = ft_gpu_execute(P->RP[0], FT_GPU_RECTDISK, 0, FT_GPU_FP64, dA, M, stream);
-        t.trans = 0;
-        if (rc == FTAMD_OK) rc = product(d, &t, dA, bytes, stream);
-        if (rc == FTAMD_OK) rc = tri_product(d, H[2], 1, 1, n, M, dA, bytes, stream);
-    } else if (!inverse) {
-        rc = tri_product(d, H[2], 1, 0, n, M, dA, bytes, stream);
-        t.trans = 1;
-        if (rc == FTAMD_OK) rc = product(d, &t, dA, bytes, stream);
-        if (rc == FTAMD_OK) rc = ft_gpu_execute(P->RP[0], FT_GPU_RECTDISK, 1, FT_GPU_FP64, dA, M, stream);
-    } else if (TRANS == 'N') {
-        rc = tri_product(d, H[2], 1, 1, n, M, dA, bytes, stream);
-        t.trans = 0;
-        if (rc == FTAMD_OK) rc = product(d, &t, dA, bytes, stream);
-        if (rc == FTAMD_OK) rc = ft_gpu_execute(P->RP[0], FT_GPU_RECTDISK, 1, FT_GPU_FP64, dA, M, stream);
-    } else {
-        rc = ft_gpu_execute(P->RP[0], FT_GPU_RECTDISK, 0, FT_GPU_FP64, dA, M, stream);
-        t.trans = 1;
-        if (rc == FTAMD_OK) rc = product(d, &t, dA, bytes, stream);
-        if (rc == FTAMD_OK) rc = tri_product(d, H[2], 1, 0, n, M, dA, bytes, stream);
-    }
+    if (fwd) rc = ft_gpu_execute(P->RP[0], FT_GPU_RECTDISK, 0, FT_GPU_FP64, dA, M, stream);
+    if (rc == FTAMD_OK) rc = products(d, p, 2, dA, bytes, stream);
+    if (rc == FTAMD_OK && !fwd) rc = ft_gpu_execute(P->RP[0], FT_GPU_RECTDISK, 1, FT_GPU_FP64, dA, M, stream);
     return rc;
 }
 
@@ -478,13 +453,14 @@ static int run_annulus(ft_harmonic_plan *P, int inverse, char TRANS, void *dA, i
     const int n = P->RP[0]->n, trans = TRANS == 'T';
     const double *H = inverse ? d->dPinv[0] : d->dP[0];
     const int rot_first = inverse ? trans : !trans;
+    FtamdTrmmLaunch t = tri_product(H, 0, trans, n, M);
     int rc = FTAMD_OK;
     if (rot_first) {
         rc = ft_gpu_execute(P->RP[0], FT_GPU_DISK, 0, FT_GPU_FP64, dA, M, stream);
         if (rc == FTAMD_OK) rc = ftamd_hip_bidiag(dA, n, M, d->dR, !inverse, trans, stream);
-        if (rc == FTAMD_OK) rc = tri_product(d, H, 0, trans, n, M, dA, bytes, stream);
+        if (rc == FTAMD_OK) rc = products(d, &t, 1, dA, bytes, stream);
     } else {
-        rc = tri_product(d, H, 0, trans, n, M, dA, bytes, stream);
+        rc = products(d, &t, 1, dA, bytes, stream);
         if (rc == FTAMD_OK) rc = ftamd_hip_bidiag(dA, n, M, d->dR, !inverse, trans, stream);
         if (rc == FTAMD_OK) rc = ft_gpu_execute(P->RP[0], FT_GPU_DISK, 1, FT_GPU_FP64, dA, M, stream);
     }

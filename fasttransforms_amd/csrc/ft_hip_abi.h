@@ -171,16 +171,15 @@ int ftamd_hip_sys_launch(const FtamdSysLaunch *a, int precision, int S, void *st
  * leading dimension n; op = identity, or the transpose when trans);
  * U[c] == NULL leaves class c out.  Right (right == 1, ncls 1, cstride 1):
  * Y = X op(U[0]) with U[0]'s leading M x M block (leading dimension n).
- * Output tiles of FTAMD_TRMM_ROWS x FTAMD_TRMM_COLS; ctiles[c] column tiles
- * per class. */
-#define FTAMD_TRMM_ROWS 64
-#define FTAMD_TRMM_COLS 32
+ * scale_in: X's entries are taken as cheb_scale(pre1, pre2) leaves them;
+ * scale_out: Y's entries are stored as cheb_scale(post1, post2) leaves them. */
 typedef struct {
     const double *U[4];
     const double *X;
     double *Y;
     int n, M, cstride, ncls, trans, right;
-    int ctiles[4];
+    int scale_in, scale_out;
+    double pre1, pre2, post1, post2;
 } FtamdTrmmLaunch;
 int ftamd_hip_trmm_launch(const FtamdTrmmLaunch *a, void *stream);
 /* Synthesis / analysis on the sphere's grid (ft_grid.hip): hipFFT plans and

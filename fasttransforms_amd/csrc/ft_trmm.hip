@@ -5,15 +5,30 @@
 //
 // Left: Y[:, j] = op(U_c) X[:, j] for every column j of every class c.
 // Right: Y = X op(U) with U's leading M x M block.  Out of place.  A
-// workgroup (4 waves) computes a 64 x 32 tile of Y: wave w the rows 16w ..
-// 16w+15 as two 16 x 16 blocks, accumulated by v_mfma_f64_16x16x4_f64 over k
-// in stages of 16 staged through LDS (the A operand 64 x 16, the B operand
-// 16 x 32), the next stage's global loads issued before the current stage's
-// products.  Lane layout of the 16x16x4 FP64 MFMA: A operand lane i =
-// A[i % 16][i / 16], B operand lane i = B[i / 16][i % 16], result register
-// j of lane i = D[i / 16 + 4 j][i % 16].  Only the triangle's k range is
-// visited.  The products sum in another order than the reference's BLAS, so
-// results agree to rounding, not bit for bit.
+// workgroup of 2 x 2 waves computes a tile of 32 rows x 32 columns of Y, a
+// wave 16 x 16 of it by v_mfma_f64_16x16x4_f64 over k in stages of 16 through
+// two LDS buffers, one barrier a stage.  Only the triangle's k range is
+// visited.  Lane layout of the 16x16x4 FP64 MFMA: A operand lane i =
+// A[i % 16][i / 16], B operand lane i = B[i / 16][i % 16], result register j
+// of lane i = D[i / 16 + 4 j][i % 16].  The operand that runs along Y's
+// columns is the A operand, so that 16 lanes hold 16 consecutive rows of one
+// column of Y (a whole 128-byte line of the store).
+//
+// What bounds it: at n = 1024, M = 2047 the matrix pipes (30 us of 50 at the
+// rate of a large product), below n = 600 the chain of stages of the longest
+// tile, some 350 clocks each, of which the products take 256.  So a stage's
+// loads are issued two stages ahead and without conditions: rows and columns
+// past the edge are clamped (their results are not stored), addresses advance
+// by one add, and the one stage that K cuts is left for the end.  One stage
+// ahead and with bounds checked at each load it was 65 us, and at n = 511 19
+// us for 11.6.  Held to 64 registers, so that eight waves share a SIMD (at 80
+// it is 56 us).  Tiles of 64 x 32 and 64 x 64 make the chain longer (17 and 27
+// us at n = 511) and are no faster at n = 1024 (49 .. 62 us).  Tiles are dealt
+// longest first and back and forth over the 256 CUs, so that a CU's
+// workgroups add up to equal work.  n = 1024, M = 2047: 74 us before (64 x 32
+// tiles, loads one stage ahead), 50 now; n = 600, M = 1199: 34, 18.
+// The products sum in another order than the reference's BLAS, so results
+// agree to rounding, not bit for bit.
 #include <hip/hip_runtime.h>
 
 #include "ft_hip_abi.h"
@@ -22,129 +37,160 @@ namespace fttrmm {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-constexpr int TR = FTAMD_TRMM_ROWS;  // output rows per workgroup
-constexpr int TC = FTAMD_TRMM_COLS;  // output columns per workgroup
-constexpr int TK = 16;               // k per stage
-constexpr int PAD = 2;               // LDS row padding (doubles)
-constexpr int NA = TR * TK / 256;    // A-operand elements each thread stages
-constexpr int NB = TK * TC / 256;    // B-operand elements each thread stages
+constexpr int TK = 16;             // k per stage
+constexpr int TR = 32, TC = 32;    // rows and columns of a tile
+constexpr int PAD = 2;             // LDS row padding (doubles): stores of 16 k x 4 columns spread over the banks
+constexpr int NE = TR * TK / 256;  // elements of each operand that a thread stages
 
-template <bool RIGHT>
-__global__ void __launch_bounds__(256) trmm_kernel(FtamdTrmmLaunch a) {
-    __shared__ double sA[TK][TR + PAD];  // sA[k][r] = A operand (r0 + r, k0 + k)
-    __shared__ double sB[TK][TC + PAD];  // sB[k][q] = B operand (k0 + k, column q of the tile)
+// Column tiles before each class, and all of them.
+struct Tiles {
+    int at[5];
+};
+
+// RIGHT, TRANS as above; SCALE: X's entries as the Chebyshev normalization
+// (cheb_scale) leaves them.
+template <bool RIGHT, bool TRANS, bool SCALE>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8, 8))) trmm_kernel(FtamdTrmmLaunch a, int rtiles, Tiles ct) {
+    __shared__ double sR[2][TK][TR + PAD];  // op(U) (left) or X (right): [k][row]
+    __shared__ double sC[2][TK][TC + PAD];  // X (left) or op(U) (right): [k][column]
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int n = a.n;
-    // class and column tile of this workgroup
-    int c = 0, t = blockIdx.x;
-    while (c + 1 < a.ncls && t >= a.ctiles[c]) t -= a.ctiles[c++];
-    const double *U = a.U[c];
-    if (U == nullptr || t >= a.ctiles[c]) return;
-    const int count = (a.M - c + a.cstride - 1) / a.cstride;  // output columns of the class
-    const int q0 = t * TC;                                    // first class-local column of the tile
-    const int r0 = blockIdx.y * TR;
-    const bool trans = a.trans != 0;
-    // k ranges of the triangle: left, rows of op(U) from r0 (U) or up to the
-    // tile's last row (U^T); right, columns of op(U) up to the tile's last
-    // column (U) or from q0 (U^T)
-    const int K = RIGHT ? a.M : n;
-    int kbeg, kend;
-    if (!RIGHT) {
-        kbeg = trans ? 0 : r0;
-        kend = trans ? min(n, r0 + TR) : n;
+    const int n = a.n, K = RIGHT ? a.M : n;
+    // the tile: by decreasing length of its k range, every other run of 256 backwards
+    int id = blockIdx.x;
+    {
+        const int total = gridDim.x, run = id & ~255, end = min(run + 256, total);
+        if (id & 256) id = run + end - 1 - id;
+    }
+    const int ctiles = ct.at[4];
+    int rt, cq;
+    if (RIGHT) {
+        const int rank = id / rtiles;
+        rt = id - rank * rtiles;
+        cq = TRANS ? rank : ctiles - 1 - rank;
     } else {
-        kbeg = trans ? q0 : 0;
-        kend = trans ? K : min(K, q0 + TC);
+        const int rank = id / ctiles;
+        cq = id - rank * ctiles;
+        rt = TRANS ? rtiles - 1 - rank : rank;
     }
-    const long long xcol = a.cstride;  // X column of class-local column q: c + q * cstride
+    int c = 0;
+    while (c < 3 && cq >= ct.at[c + 1]) ++c;
+    const double *U = a.U[c];
+    if (U == nullptr) return;
+    const int xcol = a.cstride;
+    const int count = (a.M - c + xcol - 1) / xcol;  // columns of the class
+    const int r0 = rt * TR, q0 = (cq - ct.at[c]) * TC;
+    const int kbeg = RIGHT ? (TRANS ? q0 : 0) : (TRANS ? 0 : r0);
+    const int kend = RIGHT ? (TRANS ? K : min(K, q0 + TC)) : (TRANS ? min(n, r0 + TR) : n);
+    const int kfirst = kbeg / TK * TK;
 
-    // element e of the A operand's 64 x 16 block: consecutive threads along
-    // the contiguous direction of the source
-    auto a_rk = [&](int e, int &r, int &k) {
-        const bool along_k = !RIGHT && trans;  // U^T: a column of U is a row of the operand
-        r = along_k ? e / TK : e % TR;
-        k = along_k ? e % TK : e / TR;
-    };
-    auto load_a = [&](int k0, double (&v)[NA]) {
+    // element s of the thread: (row or column, k) in the stage and its address,
+    // consecutive threads along the direction that is contiguous in memory
+    constexpr bool RK = !RIGHT && TRANS;  // op(U) = U^T from the left: contiguous in k
+    constexpr bool CK = !RIGHT || !TRANS; // X from the left, U from the right: contiguous in k
+    const double *pr[NE], *pc[NE];
+    int rr[NE], rk[NE], cc[NE], ck[NE];
 #pragma unroll
-        for (int s = 0; s < NA; ++s) {
-            int r, k;
-            a_rk(tid + 256 * s, r, k);
-            const int gr = r0 + r, gk = k0 + k;
-            double x = 0.0;
-            if (gr < n && gk < K) {
-                if (RIGHT) x = a.X[gr + (long long)gk * n];                  // X[gr][gk]
-                else x = trans ? U[gk + (long long)gr * n] : U[gr + (long long)gk * n];  // op(U)[gr][gk]
-            }
-            v[s] = x;
-        }
+    for (int s = 0; s < NE; ++s) {
+        const int e = tid + 256 * s;
+        rr[s] = RK ? e / TK : e % TR;
+        rk[s] = RK ? e % TK : e / TR;
+        cc[s] = CK ? e / TK : e % TC;
+        ck[s] = CK ? e % TK : e / TC;
+        const long long row = min(r0 + rr[s], n - 1), kr = kfirst + rk[s];
+        const long long q = min(q0 + cc[s], count - 1), kc = kfirst + ck[s];
+        pr[s] = RIGHT ? a.X + row + kr * n : TRANS ? U + kr + row * n : U + row + kr * n;
+        pc[s] = RIGHT ? (TRANS ? U + q + kc * n : U + kc + q * n) : a.X + kc + (c + q * xcol) * n;
+    }
+    const long long stepr = RK ? TK : (long long)TK * n, stepc = CK ? TK : (long long)TK * n;
+    // the normalization of X's entry (i, j)
+    auto scaled = [&](double v, int i, int j) {
+        if (!SCALE) return v;
+        if (j == 0) v *= a.pre1;
+        if (i == 0) v *= a.pre1;
+        return v * a.pre2;
     };
-    // element e of the B operand's 16 x 32 block
-    auto b_kq = [&](int e, int &k, int &q) {
-        const bool along_q = RIGHT && trans;  // U^T from the right: op(U)[k][q] = U[q][k], contiguous in q
-        k = along_q ? e / TC : e % TK;
-        q = along_q ? e % TC : e / TK;
+    struct Stage {
+        double r[NE], c[NE];
     };
-    auto load_b = [&](int k0, double (&v)[NB]) {
+    auto load = [&](Stage &v, bool advance) {  // and on to the next stage
 #pragma unroll
-        for (int s = 0; s < NB; ++s) {
-            int k, q;
-            b_kq(tid + 256 * s, k, q);
-            const int gk = k0 + k, gq = q0 + q;
-            double x = 0.0;
-            if (gk < K && gq < count) {
-                if (RIGHT) x = trans ? U[gq + (long long)gk * n] : U[gk + (long long)gq * n];  // op(U)[gk][gq]
-                else x = a.X[gk + (c + gq * xcol) * n];                                        // X[gk][column]
-            }
-            v[s] = x;
-        }
+        for (int s = 0; s < NE; ++s) v.r[s] = *pr[s];
+#pragma unroll
+        for (int s = 0; s < NE; ++s) v.c[s] = *pc[s];
+        const long long ar = advance ? stepr : 0, ac = advance ? stepc : 0;
+#pragma unroll
+        for (int s = 0; s < NE; ++s) pr[s] += ar, pc[s] += ac;
     };
-    auto store = [&](const double (&va)[NA], const double (&vb)[NB]) {
+    auto store = [&](const Stage &v, int buf, int k0) {
 #pragma unroll
-        for (int s = 0; s < NA; ++s) {
-            int r, k;
-            a_rk(tid + 256 * s, r, k);
-            sA[k][r] = va[s];
-        }
+        for (int s = 0; s < NE; ++s) sR[buf][rk[s]][rr[s]] = RIGHT ? scaled(v.r[s], r0 + rr[s], k0 + rk[s]) : v.r[s];
 #pragma unroll
-        for (int s = 0; s < NB; ++s) {
-            int k, q;
-            b_kq(tid + 256 * s, k, q);
-            sB[k][q] = vb[s];
-        }
+        for (int s = 0; s < NE; ++s)
+            sC[buf][ck[s]][cc[s]] = RIGHT ? v.c[s] : scaled(v.c[s], k0 + ck[s], c + (q0 + cc[s]) * xcol);
     };
 
-    v4d acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
-    double va[NA], vb[NB];
-    const int k_first = kbeg / TK * TK;
-    if (k_first < kend) {
-        load_a(k_first, va);
-        load_b(k_first, vb);
-    }
-    for (int k0 = k_first; k0 < kend; k0 += TK) {
-        store(va, vb);
+    const int wr = (w & 1) * 16 + (lane & 15), wc = (w >> 1) * 16 + (lane & 15), wk = lane >> 4;
+    v4d acc = {0, 0, 0, 0};
+    auto multiply = [&](int buf) {
+#pragma unroll
+        for (int ks = 0; ks < TK; ks += 4)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(sC[buf][ks + wk][wc], sR[buf][ks + wk][wr], acc, 0, 0, 0);
+    };
+    // Full stages kfirst + TK i, i < full, and a last one that K cuts.
+    const int full = (min(kend, K / TK * TK) - kfirst + TK - 1) / TK, klast = kfirst + full * TK;
+    Stage v0, v1;
+    if (full > 0) {
+        load(v0, full > 1);
+        load(v1, full > 2);
+        store(v0, 0, kfirst);
         __syncthreads();
-        // the next stage's loads are in flight during this stage's products
-        if (k0 + TK < kend) {
-            load_a(k0 + TK, va);
-            load_b(k0 + TK, vb);
+        // stage i in buffer i % 2; the loads of stage i + 2 (past the end: of the
+        // last one again) are issued before its products, those of stage i + 1,
+        // issued a stage earlier, stored after them
+        for (int i = 0; i < full; i += 2) {
+            load(v0, i + 3 < full);
+            multiply(0);
+            store(v1, 1, kfirst + (i + 1) * TK);
+            __syncthreads();
+            if (i + 1 == full) break;
+            load(v1, i + 4 < full);
+            multiply(1);
+            store(v0, 0, kfirst + (i + 2) * TK);
+            __syncthreads();
+        }
+    }
+    if (klast < kend) {  // zeros past K; the addresses stand at the last full stage
+        const long long ar = full > 0 ? stepr : 0, ac = full > 0 ? stepc : 0;
+#pragma unroll
+        for (int s = 0; s < NE; ++s) {
+            const bool in = klast + rk[s] < K;
+            const double x = *(in ? pr[s] + ar : a.X);
+            v0.r[s] = in ? x : 0.0;
         }
 #pragma unroll
-        for (int ks = 0; ks < TK; ks += 4) {
-            const int kk = ks + (lane >> 4), ii = lane & 15;
-            const double av = sA[kk][16 * w + ii];
-            acc0 = __builtin_amdgcn_mfma_f64_16x16x4f64(av, sB[kk][ii], acc0, 0, 0, 0);
-            acc1 = __builtin_amdgcn_mfma_f64_16x16x4f64(av, sB[kk][16 + ii], acc1, 0, 0, 0);
+        for (int s = 0; s < NE; ++s) {
+            const bool in = klast + ck[s] < K;
+            const double x = *(in ? pc[s] + ac : a.X);
+            v0.c[s] = in ? x : 0.0;
         }
+        store(v0, 0, klast);
         __syncthreads();
+        multiply(0);
     }
+    const int r = r0 + wr;
+    if (r >= n) return;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        const int r = r0 + 16 * w + (lane >> 4) + 4 * j;
-        if (r >= n) continue;
-        const int qa = q0 + (lane & 15), qb = qa + 16;
-        if (qa < count) a.Y[r + (c + qa * xcol) * n] = acc0[j];
-        if (qb < count) a.Y[r + (c + qb * xcol) * n] = acc1[j];
+    for (int e = 0; e < 4; ++e) {
+        const int q = q0 + (w >> 1) * 16 + wk + 4 * e;
+        if (q >= count) continue;
+        const int col = c + q * xcol;
+        double v = acc[e];
+        if (a.scale_out) {  // cheb_scale
+            if (col == 0) v *= a.post1;
+            if (r == 0) v *= a.post1;
+            v *= a.post2;
+        }
+        a.Y[r + (long long)col * n] = v;
     }
 }
 
@@ -288,19 +334,33 @@ extern "C" int ftamd_hip_bidiag(double *A, int n, int M, const double *R, int so
     return e == hipSuccess ? FTAMD_OK : FTAMD_EDEVICE;
 }
 
+namespace {
+
+template <bool RIGHT, bool TRANS, bool SCALE> void launch(const FtamdTrmmLaunch &a, hipStream_t st) {
+    using namespace fttrmm;
+    Tiles ct;
+    ct.at[0] = 0;
+    for (int c = 0; c < 4; ++c) {
+        const int count = c < a.ncls && a.M > c ? (a.M - c + a.cstride - 1) / a.cstride : 0;
+        ct.at[c + 1] = ct.at[c] + (count + TC - 1) / TC;
+    }
+    const int rtiles = (a.n + TR - 1) / TR;
+    hipLaunchKernelGGL((trmm_kernel<RIGHT, TRANS, SCALE>), dim3(ct.at[4] * rtiles), dim3(256), 0, st, a, rtiles, ct);
+}
+
+template <bool RIGHT> void launch_side(const FtamdTrmmLaunch &a, hipStream_t st) {
+    if (a.trans) a.scale_in ? launch<RIGHT, true, true>(a, st) : launch<RIGHT, true, false>(a, st);
+    else a.scale_in ? launch<RIGHT, false, true>(a, st) : launch<RIGHT, false, false>(a, st);
+}
+
+}  // namespace
+
 extern "C" int ftamd_hip_trmm_launch(const FtamdTrmmLaunch *a, void *stream) {
     if (a->n < 1 || a->M < 0 || a->cstride < 1 || a->ncls < 1 || a->ncls > 4 || !a->X || !a->Y) return FTAMD_EINVAL;
     if (a->right && (a->ncls != 1 || a->cstride != 1 || a->M > a->n)) return FTAMD_EINVAL;
-    int tiles = 0;
-    for (int c = 0; c < a->ncls; ++c) {
-        const int count = a->M > c ? (a->M - c + a->cstride - 1) / a->cstride : 0;
-        if (a->ctiles[c] != (count + FTAMD_TRMM_COLS - 1) / FTAMD_TRMM_COLS) return FTAMD_EINVAL;
-        tiles += a->ctiles[c];
-    }
-    const int rows = (a->n + FTAMD_TRMM_ROWS - 1) / FTAMD_TRMM_ROWS;
-    if (tiles == 0) return FTAMD_OK;
-    if (a->right) hipLaunchKernelGGL(fttrmm::trmm_kernel<true>, dim3(tiles, rows), dim3(256), 0, (hipStream_t)stream, *a);
-    else hipLaunchKernelGGL(fttrmm::trmm_kernel<false>, dim3(tiles, rows), dim3(256), 0, (hipStream_t)stream, *a);
+    if (a->M == 0) return FTAMD_OK;
+    if (a->right) launch_side<true>(*a, (hipStream_t)stream);
+    else launch_side<false>(*a, (hipStream_t)stream);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FTAMD_OK : (e == hipErrorOutOfMemory ? FTAMD_ENOMEM : FTAMD_EDEVICE);
 }
