@@ -7,16 +7,21 @@
 // the opposite order.  The real and imaginary parts take the same real
 // rotation.
 //
-// Two lanes own a complex column, one its real and one its imaginary part,
-// and sweep its sequences one after another down (hi2lo) or up (lo2hi) the
-// column: a step rotates the fresh row against the carried one and emits a
-// finished row.  The launch has few waves (one per 32 parts of columns), so
-// a step's cost is its instructions issued in order plus the carried row's
-// FP64 latency; the sweep keeps a step to one rotation (no per-step range
-// bookkeeping: every pair of a sequence is in its range) and loads the next
-// block of rows and (s, c) while the current block is computed.  (A
-// systolic sweep of up to 8 sequences per lane, complex columns per lane,
-// measured slower at every spin.)
+// A wave owns four columns and takes up to four of their sequences at a time:
+// a lane for each sequence and real or imaginary part, which sweeps down
+// (hi2lo) or up (lo2hi) the column in blocks of 16 rows, a step rotating the
+// fresh row against the carried one and emitting a finished row.  A
+// sequence's lane is a block behind the one before it and takes the rows that
+// this one emitted from LDS.  All 64 lanes move data: a block is one 16-byte
+// load a lane of rows and one of (s, c) for each sequence, two blocks ahead,
+// passed on through LDS, and one store.
+//
+// What bounds it: the instructions of a step (four FP64, two LDS reads),
+// issued in order by the one wave of a SIMD.  Loads by the computing lanes
+// themselves (32 columns a wave, each lane its own line, one block of 12 rows
+// ahead, one sequence a sweep) took 146 clocks a step and sequence, waiting
+// for memory; two sequences in one lane take 26 us.  n = 512, s = 2: 68 us
+// before, 22 now.
 //
 // The transpose of the rotation (s, c) is the rotation (-s, c), bit for bit
 // in the fused forms: fma(c, x, (-s)*y) = fma(c, x, -(s*y)) and
@@ -31,93 +36,175 @@ namespace ftspin {
 __device__ __forceinline__ double rot_x(double C, double S, double x, double y) { return __builtin_fma(C, x, S * y); }
 __device__ __forceinline__ double rot_y(double C, double S, double x, double y) { return __builtin_fma(C, y, -(S * x)); }
 
-// One sequence over one part of a column: the pairs are r = R-1 .. 0 (hi2lo) or 0 .. R-1
-// (lo2hi), every one of them in the sequence's range, so a step is one
-// rotation of the fresh row against the carried one, emitting a finished
-// row.  Full blocks of KB steps run without a branch, the next block's rows
-// and (s, c) loaded at clamped indices while this one is computed; the
-// remaining R mod KB steps and the last row follow.
-template <int DIR>
-__device__ void sweep1(double *col, long long rs, const double2 *__restrict__ tq, int R, double sg) {
-    using V = double;
-    constexpr int KB = 12;
-    // step p = 1 .. R: the fresh row and the pair, clamped into range past R
-    auto frow = [&](int p) {
-        const int pc = p > R ? R : p;
-        return DIR == 0 ? R - pc : pc;
+constexpr int CW = 4;   // columns of a wave
+constexpr int KB = 16;  // elements of a block
+constexpr int PITCH = KB + 1;
+constexpr int MAXS = 4;  // most sequences at a time
+
+struct Column {
+    int R;            // last row of sequence 0
+    int nrot;         // its sequences; 0 past the last column
+    long long base;   // its row 0 (complex entries from A)
+    long long tab;    // sequence 0's (s, c)
+    double sg;        // sign of s
+};
+
+struct Args {
+    const double2 *tab;
+    int n, s;
+    double2 *A;
+    int c0, count;
+    long long col_stride;
+    int row_stride, use_fixed, fixed_m, dir;
+    int nlow, low_blocks;  // the first nlow columns have waves of their own, low_blocks of them
+};
+
+// The wave's column of a slot.  The first nlow columns are of orders |m| < |s|,
+// with |m| sequences: wave k - 1 takes orders -k and k.
+__device__ Column column(const Args &a, int slot) {
+    int c;
+    bool in;
+    if ((int)blockIdx.x < a.low_blocks) {
+        c = 2 * (int)blockIdx.x + 1 + slot;
+        in = slot < 2 && c >= a.c0 && c < a.c0 + a.nlow;
+    } else {
+        c = a.c0 + a.nlow + ((int)blockIdx.x - a.low_blocks) * CW + slot;
+        in = c < a.c0 + a.count;
+    }
+    if (!in) c = a.c0;
+    const int m = a.use_fixed ? a.fixed_m : ((c & 1) ? -((c + 1) >> 1) : (c >> 1));
+    const int as = a.s < 0 ? -a.s : a.s, am = m < 0 ? -m : m;
+    const int d = am > as ? am - as : as - am;
+    const int nseq = am < as ? am : as;
+    Column q;
+    q.R = a.n - 1 - d;
+    q.nrot = in ? max(0, min(nseq, q.R)) : 0;
+    q.base = a.col_stride * (c - a.c0);
+    q.tab = (long long)d * as * a.n;
+    q.sg = (a.dir == 0) == ((m >= 0) == (a.s >= 0)) ? 1.0 : -1.0;
+    return q;
+}
+
+__device__ int wave_max(int v) {
+    for (int k = 32; k; k >>= 1) v = max(v, __shfl_xor(v, k));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+
+struct Shared {
+    double2 rows[MAXS + 1][CW * PITCH];  // [s]: the rows that stage s takes, [s + 1]: those it emitted
+    double2 sc[MAXS][CW * PITCH];
+};
+
+// The sequences jl .. jl + S - 1 over the wave's columns: lq the column whose
+// data this lane moves, cq the one it computes on.  Stage st is sequence jl +
+// S - 1 - st (hi2lo) or jl + st (lo2hi).  Element t of a column is row RL - t
+// (t), RL the last row of sequence jl: a stage takes element t and emits
+// element t - 1, rotated by the sequence's pair RL - t (t - 1) if it has that,
+// else as it is; so nothing but t tells the first and the last steps apart.
+// In round g stage st takes elements 16 (g - st) - st and up.
+template <int DIR, int S>
+__device__ void sweep(const Args &a, const Column &lq, const Column &cq, int jl, Shared &sh) {
+    const int lane = threadIdx.x, lcol = lane / KB, lk = lane % KB;
+    const int h = lane & 1, ccol = (lane >> 1) & (CW - 1), st = lane / (2 * CW);
+    const bool lvalid = jl < lq.nrot, cvalid = jl < cq.nrot;
+    const int RL = lvalid ? lq.R - jl : 0, RC = cvalid ? cq.R - jl : 0;
+    const int rounds = (wave_max(RC) + S) / KB + S;
+    const int full = -wave_max(cvalid ? -RC : -(1 << 30));  // every column has elements up to here
+    const int act0 = DIR == 0 ? S - st : 1, act1 = DIR == 0 ? RC : RC - st;
+    const double2 *lt = a.tab + (lvalid ? lq.tab + (long long)jl * a.n : 0);
+    double2 *lA = a.A + lq.base;
+    struct Block {
+        double2 x, sc[S];
     };
-    auto pair = [&](int p) {
-        const int pc = p > R ? R : p;
-        return DIR == 0 ? R - pc : pc - 1;
-    };
-    auto load = [&](int p0, V (&x)[KB], double2 (&sc)[KB]) {
+    auto load = [&](Block &v, int g) {
+        const int t = max(0, min(g * KB + lk, RL));
+        v.x = lA[(long long)(DIR == 0 ? RL - t : t) * a.row_stride];
 #pragma unroll
-        for (int k = 0; k < KB; ++k) {
-            x[k] = col[(long long)frow(p0 + k) * rs];
-            sc[k] = tq[pair(p0 + k)];
+        for (int s = 0; s < S; ++s) {
+            const int j = lvalid ? (DIR == 0 ? S - 1 - s : s) : 0, ts = (g - s) * KB - s + lk;
+            const int pair = DIR == 0 ? RL - ts : ts - 1;
+            v.sc[s] = lt[(long long)j * a.n + max(0, min(pair, RL - j - 1))];
         }
     };
-    // hi2lo: x row r, the carry row r+1, emits row r+1; lo2hi: the carry row r, x row r+1, emits row r
-    auto step = [&](V x, double2 sc, V &cy) {
-        const double S = sg * sc.x, C = sc.y;
-        V em;
-        if (DIR == 0) {
-            em = rot_y(C, S, x, cy);
-            cy = rot_x(C, S, x, cy);
-        } else {
-            em = rot_x(C, S, cy, x);
-            cy = rot_y(C, S, cy, x);
+    // in this order, so that a wait for one block's loads is none for the next one's
+    Block v0, v1;
+    __builtin_amdgcn_sched_barrier(0);
+    load(v0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(v1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+
+    double cy = 0.0;
+    auto rotate = [&](double2 sc, double x) {
+        double em;
+        if (DIR == 0) {  // x row r, the carried row r + 1, emits row r + 1
+            em = rot_y(sc.y, sc.x, x, cy);
+            cy = rot_x(sc.y, sc.x, x, cy);
+        } else {  // the carried row r, x row r + 1, emits row r
+            em = rot_x(sc.y, sc.x, cy, x);
+            cy = rot_y(sc.y, sc.x, cy, x);
         }
         return em;
     };
-    auto out_row = [&](int p) { return (long long)(DIR == 0 ? R - p + 1 : p - 1) * rs; };
-    V cy = col[(long long)(DIR == 0 ? R : 0) * rs];
-    const int nb = R / KB;
-    V xb[KB], xn[KB];
-    double2 sb[KB], sn[KB];
-    load(1, xb, sb);
-    for (int b = 0; b < nb; ++b) {
-        const int p0 = 1 + b * KB;
-        load(p0 + KB, xn, sn);
+    auto round = [&](int g, Block &v) {
+        sh.rows[0][lcol * PITCH + lk] = v.x;
 #pragma unroll
-        for (int k = 0; k < KB; ++k) col[out_row(p0 + k)] = step(xb[k], sb[k], cy);
+        for (int s = 0; s < S; ++s) sh.sc[s][lcol * PITCH + lk] = make_double2(lq.sg * v.sc[s].x, v.sc[s].y);
+        load(v, g + 2);
+        __syncthreads();
+        if (lane < 2 * CW * S) {
+            const double2 *in = &sh.rows[st][ccol * PITCH], *csc = &sh.sc[st][ccol * PITCH];
+            double *out = (double *)&sh.rows[st + 1][ccol * PITCH] + h;
+            double x[KB];
+            double2 sc[KB];
 #pragma unroll
-        for (int k = 0; k < KB; ++k) {
-            xb[k] = xn[k];
-            sb[k] = sn[k];
+            for (int k = 0; k < KB; ++k) {
+                x[k] = ((const double *)&in[k])[h];
+                sc[k] = csc[k];
+            }
+            if (g >= S && g * KB + KB - 1 <= full) {
+#pragma unroll
+                for (int k = 0; k < KB; ++k) out[2 * k] = rotate(sc[k], x[k]);
+            } else {
+                const int t0 = (g - st) * KB - st;
+#pragma unroll
+                for (int k = 0; k < KB; ++k) {
+                    const bool act = t0 + k >= act0 && t0 + k <= act1;
+                    const double c0 = cy, em = rotate(sc[k], x[k]);
+                    if (!act) cy = x[k];
+                    out[2 * k] = act ? em : c0;
+                }
+            }
         }
+        __syncthreads();
+        const int t = (g - S + 1) * KB - S + lk;
+        if (lvalid && t >= 0 && t <= RL)
+            lA[(long long)(DIR == 0 ? RL - t : t) * a.row_stride] = sh.rows[S][lcol * PITCH + lk];
+    };
+    for (int g = 0; g < rounds; g += 2) {  // a round past the end stores nothing
+        round(g, v0);
+        round(g + 1, v1);
     }
-    const int p0 = 1 + nb * KB, rem = R - nb * KB;
-#pragma unroll
-    for (int k = 0; k < KB; ++k)
-        if (k < rem) col[out_row(p0 + k)] = step(xb[k], sb[k], cy);
-    col[(long long)(DIR == 0 ? 0 : R) * rs] = cy;
+    __threadfence_block();  // the next sweep's loads take rows that other lanes stored
+    __syncthreads();
 }
 
-// One sequence a sweep (sweep1), two lanes a complex column (lane 2i + h
-// owns part h of column i): R = n-1-d-j0, (s, c) of sequence j0.
-__global__ void __launch_bounds__(64) stage1_split_kernel(const double2 *__restrict__ tab, int n, int s, double2 *A,
-                                                          int c0, int count, long long col_stride, int row_stride,
-                                                          int use_fixed, int fixed_m, int dir) {
-    const int l = blockIdx.x * blockDim.x + threadIdx.x;
-    const int i = l >> 1, h = l & 1;
-    if (i >= count) return;
-    const int c = c0 + i;
-    const int m = use_fixed ? fixed_m : ((c & 1) ? -((c + 1) >> 1) : (c >> 1));
-    const int as = s < 0 ? -s : s, am = m < 0 ? -m : m;
-    const int nseq = am < as ? am : as;
-    const int d = am > as ? am - as : as - am;
-    if (nseq == 0 || n - 2 - d < 0) return;
-    const int nrot = nseq < n - 1 - d ? nseq : n - 1 - d;
-    const bool rot = (m >= 0) == (s >= 0);
-    const double sg = (dir == 0) == rot ? 1.0 : -1.0;
-    double *col = (double *)(A + col_stride * i) + h;
-    const long long rs = 2LL * row_stride;
-    const double2 *t = tab + (long long)d * as * n;
-    if (dir == 0) {
-        for (int j0 = nrot - 1; j0 >= 0; --j0) sweep1<0>(col, rs, t + (long long)j0 * n, n - 1 - d - j0, sg);
+template <int DIR> __global__ void __launch_bounds__(64) stage1_kernel(Args a) {
+    __shared__ Shared sh;
+    const int lane = threadIdx.x;
+    const Column lq = column(a, lane / KB), cq = column(a, (lane >> 1) & (CW - 1));
+    const int most = wave_max(cq.nrot), least = -wave_max(cq.nrot > 0 ? -cq.nrot : -(1 << 30));
+    // several sequences at a time where the columns have the same number of them
+    const int fours = most == least ? most / 4 : 0, twos = most == least ? (most - 4 * fours) / 2 : 0;
+    const int single = 4 * fours + 2 * twos;
+    if (DIR == 0) {
+        for (int j = most - 1; j >= single; --j) sweep<0, 1>(a, lq, cq, j, sh);
+        if (twos) sweep<0, 2>(a, lq, cq, 4 * fours, sh);
+        for (int j = fours - 1; j >= 0; --j) sweep<0, 4>(a, lq, cq, 4 * j, sh);
     } else {
-        for (int j0 = 0; j0 < nrot; ++j0) sweep1<1>(col, rs, t + (long long)j0 * n, n - 1 - d - j0, sg);
+        for (int j = 0; j < fours; ++j) sweep<1, 4>(a, lq, cq, 4 * j, sh);
+        if (twos) sweep<1, 2>(a, lq, cq, 4 * fours, sh);
+        for (int j = single; j < most; ++j) sweep<1, 1>(a, lq, cq, j, sh);
     }
 }
 
@@ -130,14 +217,29 @@ extern "C" int ftamd_hip_spin_stage1(const double *tab2, int n, int s, double *A
         return FTAMD_EINVAL;
     if (count == 0 || s == 0) return FTAMD_OK;
     if (!tab2) return FTAMD_EINVAL;
-    if (count > (1 << 29)) return FTAMD_EINVAL;  // two lanes a column, lane indices in an int
-    const int block = 64;
-    const dim3 grid((2 * count + block - 1) / block);
-    const hipStream_t st = (hipStream_t)stream;
-    const double2 *tab = (const double2 *)tab2;
-    double2 *a = (double2 *)A;
-    hipLaunchKernelGGL(ftspin::stage1_split_kernel, grid, dim3(block), 0, st, tab, n, s, a, c0, count, col_stride,
-                       row_stride, use_fixed, fixed_m, dir);
+    if (count > (1 << 29)) return FTAMD_EINVAL;
+    const int as = s < 0 ? -s : s;
+    // columns of orders |m| < |s|, c < 2 |s| - 1, have |m| sequences, the others |s|
+    const long long low = use_fixed ? 0 : 2LL * as - 1 - c0;
+    ftspin::Args a;
+    a.tab = (const double2 *)tab2;
+    a.n = n;
+    a.s = s;
+    a.A = (double2 *)A;
+    a.c0 = c0;
+    a.count = count;
+    a.col_stride = col_stride;
+    a.row_stride = row_stride;
+    a.use_fixed = use_fixed;
+    a.fixed_m = fixed_m;
+    a.dir = dir;
+    a.nlow = low < 0 ? 0 : low < count ? (int)low : count;
+    a.low_blocks = a.nlow > 0 ? (c0 + a.nlow) / 2 : 0;  // orders 1 .. that of the last of them
+    const int blocks = a.low_blocks + (count - a.nlow + ftspin::CW - 1) / ftspin::CW;
+    if (blocks == 0) return FTAMD_OK;  // order 0 alone
+    const dim3 grid(blocks), block(64);
+    if (dir == 0) hipLaunchKernelGGL(ftspin::stage1_kernel<0>, grid, block, 0, (hipStream_t)stream, a);
+    else hipLaunchKernelGGL(ftspin::stage1_kernel<1>, grid, block, 0, (hipStream_t)stream, a);
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FTAMD_OK : FTAMD_EDEVICE;
 }
