@@ -208,8 +208,8 @@ struct Engine {
                      : "v"(lane16), "s"(src_base), "v"(after), "n"(K * kStepBytes)
                      : "memory");
     }
-    // A DMA of a dword a lane from the start of the tables to nowhere in particular.
-    __device__ static void dma_filler(Shared &sh, const void *tab, unsigned lane16) {
+    // A DMA of a dword a lane from the start of a table to nowhere in particular.
+    __device__ static void dma_filler(Shared &sh, const char *tab, unsigned lane16) {
         asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
                      :
                      : "s"(uniform((int)lds_addr(sh.spare))), "v"(lane16), "s"(tab)
@@ -548,6 +548,11 @@ struct Engine {
 
         const unsigned m0_base = uniform(lds_addr(&sh.scr[g][0][0]));
         const int total = (slots + kLag + kU) & ~(kU - 1);  // the last position is stored in step slots + kLag
+        // the last block of the table (identities, as all past the band's
+        // steps): FP32 reads two blocks ahead, past the table's end at the last
+        // steps, and takes this one there; FP64's one stays inside
+        const int t_tab = uniform(band->steps) + FTAMD_SYS_PREFETCH - kU + off;
+        static_assert(kD > kU || kLag + kU + kD <= kOutDelay + 1 + FTAMD_SYS_PREFETCH, "table reads past the table");
         const int in_free_end = in_base + span(R, off);
         constexpr unsigned kSlotBytes = sizeof(Pair<T>[kRows]);
         const unsigned in_lane = in_lds + (unsigned)r * (unsigned)sizeof(Pair<T>);
@@ -580,11 +585,11 @@ struct Engine {
 #pragma unroll
                     for (int q = 0; q < kU; q += kRowsDma) {
                         if (q == 0 || p0 + q < npa) dma_rows(p0 + q);
-                        else dma_filler(sh, a.tab, lane16);
+                        else dma_filler(sh, tab_band, lane16);
                     }
                 } else {
 #pragma unroll
-                    for (int q = 0; q < kU; q += kRowsDma) dma_filler(sh, a.tab, lane16);
+                    for (int q = 0; q < kU; q += kRowsDma) dma_filler(sh, tab_band, lane16);
                 }
             }
             // the addresses of the block's LDS accesses: ring slots of the
@@ -593,7 +598,8 @@ struct Engine {
             const unsigned tab0 = kD == kU ? 0u : (unsigned)(t0 % kD) * kStepBytes;
             const unsigned tab1 = kD == kU ? 0u : (unsigned)((t0 + kU) % kD) * kStepBytes;
             set_m0(m0_base + tab0);
-            const char *src = tab_band + (long long)(t0 + kD) * kStepBytes;  // step t0+kD+K: the DMA of step u, K = u+1-kSPD
+            // step t0+kD+K: the DMA of step u, K = u+1-kSPD
+            const char *src = tab_band + (long long)(kD > kU ? min(t0 + kD, t_tab) : t0 + kD) * kStepBytes;
             const unsigned pin_next = in_lane + ((unsigned)(t0 + kU) % kZ) * kSlotBytes;
 #pragma unroll
             for (int u = 0; u < kU; ++u) {
@@ -661,7 +667,7 @@ struct Engine {
                 } else {
                     *lds_at<T>(out_lane + ((unsigned)t0 + out_slot0) % kZ * kSlotBytes) = v;
                     pub_avail = out_base + (t0 + kU - kLag - off) + out_off;
-                    if (END & kLast) dma_filler(sh, a.tab, lane16);
+                    if (END & kLast) dma_filler(sh, tab_band, lane16);
                 }
             } else {
                 const int po0 = t0 - kLag - off, po = po0 + out_u;
@@ -678,7 +684,7 @@ struct Engine {
                     pub = max(0, min(po0 + kU, R + 1));
                 }
                 // unless some lane stored a row of A
-                if (END & kLast && max(max(po0, ring_hi + 1), 0) > min(po0 + kU - 1, R)) dma_filler(sh, a.tab, lane16);
+                if (END & kLast && max(max(po0, ring_hi + 1), 0) > min(po0 + kU - 1, R)) dma_filler(sh, tab_band, lane16);
             }
             out_a += astep * kU;
             t0 += kU;

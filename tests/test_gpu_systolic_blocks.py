@@ -34,3 +34,25 @@ def test_block_edges(ft, kind, params, precision, maxpart):
     finally:
         ft.set_engine(ft.ENGINE_AUTO)
         ft.set_systolic(0)
+
+
+@pytest.mark.parametrize("kind,params,n", [("sph", (), 128), ("sph", (), 256), ("tri", (0.0, 0.0, 0.0), 64),
+                                           ("disk", (0.0, 0.0), 64), ("disk", (0.0, 0.0), 128)])
+@pytest.mark.parametrize("d", [0, 1])
+def test_tables_that_end_with_their_page(ft, kind, params, n, d):
+    """FP32 tables whose last byte is the last of a 4 KB page: what the last
+    steps read ahead is still inside them."""
+    import torch
+    plan = {"sph": ft.plan_rotsphere, "tri": ft.plan_rottriangle, "disk": ft.plan_rotdisk}[kind]
+    M = {"sph": 2 * n - 1, "tri": n, "disk": 4 * n - 3}[kind]
+    ft.set_engine(ft.ENGINE_SYSTOLIC)
+    try:
+        P, Q = plan(n, *params), O.Plan(kind, n, *params)
+        A = O.fill(kind, n, M, n).astype(np.float32).copy(order="F")
+        T = torch.from_numpy(np.ascontiguousarray(A.T)).cuda()
+        print("page end", kind, n, d, flush=True)
+        ft.gpu_execute(P, d, T, M=M, precision=1)
+        ft.synchronize()
+        assert np.array_equal(T.cpu().numpy().T, O.execute_f32(Q, d, A.copy(order="F"), M))
+    finally:
+        ft.set_engine(ft.ENGINE_AUTO)
