@@ -1657,97 +1657,145 @@ void ft_kernel_spinsph_lo2hi(const ft_spin_rotation_plan *P, const int m, ft_com
  * go into the per-XCD, pass-ordered lists, so small transforms fill in around
  * the long chains of the large ones.
  *
- * The schedule of the last argument list is cached.  It is keyed on the whole
- * list, compared entry by entry: every plan pointer with the plan's serial
+ * The schedules of the last FTAMD_BATCHES argument lists are cached (a program
+ * that works on several batches in turn would else build each again on every
+ * call, 1.5 ms for 48 spheres of degree 32 .. 512 that run in 0.2; eight take
+ * about a megabyte each).  One is keyed on the whole list, compared entry by
+ * entry: every plan pointer with the plan's serial
  * number (a plan created at a freed plan's address gets another serial) and
  * n, every matrix pointer and M, plus kind, direction, precision, engine and
- * tuning (L, W and the band-systolic part size).  Destroying a plan the cached schedule uses drops the schedule.
+ * tuning (L, W and the band-systolic part size).  Destroying
+ * a plan that a cached schedule uses drops the schedule, and the least recently
+ * used one makes room for a new list.
+ *
+ * Where only the matrices differ, a band-systolic schedule is kept and its
+ * chains get the new matrices' offsets by a small kernel before the launch (48
+ * spheres of degree 32 .. 512: 1.3 ms of host work to build the schedule
+ * again, 5 us for the kernel), which waits for the schedule's last launch on
+ * whatever stream.  A stream under capture, and any call after a launch was
+ * captured (a graph may run at any time), builds a schedule as for new sizes.
  */
+#define FTAMD_BATCHES 8
+
 typedef struct {
-    pthread_mutex_t lock;
     ft_schedule *sched;
+    unsigned long long used; /* the call that last used it */
     int count, kind, dir, precision, L, W, engine, part;
     const ft_rotation_plan **plans;
     unsigned long long *serial;
     int *n;
     void **dA;
     int *M;
+    void *event;  /* after the schedule's last launch */
+    int captured; /* a launch of it was captured, or is not behind the event */
 } ft_batch_cache;
 
-static ft_batch_cache g_batch = {PTHREAD_MUTEX_INITIALIZER, NULL, 0, 0, 0, 0, 0, 0, 0, 0, NULL, NULL, NULL, NULL, NULL};
+static pthread_mutex_t g_batch_lock = PTHREAD_MUTEX_INITIALIZER;
+static ft_batch_cache g_batches[FTAMD_BATCHES];
+static unsigned long long g_batch_calls = 0;
 
-static void batch_cache_clear_locked(void) {
-    if (g_batch.sched) {
+static void batch_cache_clear_locked(ft_batch_cache *B) {
+    if (B->sched) {
         ftamd_hip_sync(NULL);
-        ftamd_schedule_release(g_batch.sched);
+        ftamd_schedule_release(B->sched);
     }
-    g_batch.sched = NULL;
-    free(g_batch.plans);
-    free(g_batch.serial);
-    free(g_batch.n);
-    free(g_batch.dA);
-    free(g_batch.M);
-    g_batch.plans = NULL;
-    g_batch.serial = NULL;
-    g_batch.n = NULL;
-    g_batch.dA = NULL;
-    g_batch.M = NULL;
-    g_batch.count = 0;
+    B->sched = NULL;
+    free(B->plans);
+    free(B->serial);
+    free(B->n);
+    free(B->dA);
+    free(B->M);
+    B->plans = NULL;
+    B->serial = NULL;
+    B->n = NULL;
+    B->dA = NULL;
+    B->M = NULL;
+    ftamd_hip_event_destroy(B->event);
+    B->event = NULL;
+    B->captured = 0;
+    B->count = 0;
 }
 
 void ftamd_batch_forget_plan(const ft_rotation_plan *RP) {
-    pthread_mutex_lock(&g_batch.lock);
-    for (int i = 0; g_batch.sched && i < g_batch.count; i++)
-        if (g_batch.plans[i] == RP && g_batch.serial[i] == RP->serial) {
-            batch_cache_clear_locked();
-            break;
-        }
-    pthread_mutex_unlock(&g_batch.lock);
+    pthread_mutex_lock(&g_batch_lock);
+    for (int k = 0; k < FTAMD_BATCHES; k++) {
+        ft_batch_cache *B = &g_batches[k];
+        for (int i = 0; B->sched && i < B->count; i++)
+            if (B->plans[i] == RP && B->serial[i] == RP->serial) {
+                batch_cache_clear_locked(B);
+                break;
+            }
+    }
+    pthread_mutex_unlock(&g_batch_lock);
 }
 
-static int batch_cache_hit(const ft_rotation_plan *const *plans, int kind, int direction, int precision,
-                           void *const *dA, const int *M, int count, int L, int W, int engine, int part) {
-    if (!g_batch.sched || g_batch.count != count || g_batch.kind != kind || g_batch.dir != direction ||
-        g_batch.precision != precision || g_batch.L != L || g_batch.W != W || g_batch.engine != engine ||
-        g_batch.part != part)
+/* Whether a cached schedule is one of these plans, sizes and choices; sets
+ * *same to whether it is of these matrices. */
+static int batch_cache_hit(const ft_batch_cache *B, const ft_rotation_plan *const *plans, int kind, int direction, int precision,
+                           void *const *dA, const int *M, int count, int L, int W, int engine, int part,
+                           int *same) {
+    *same = 1;
+    if (!B->sched || B->count != count || B->kind != kind || B->dir != direction ||
+        B->precision != precision || B->L != L || B->W != W || B->engine != engine ||
+        B->part != part)
         return 0;
-    for (int i = 0; i < count; i++)
-        if (g_batch.plans[i] != plans[i] || g_batch.serial[i] != plans[i]->serial || g_batch.n[i] != plans[i]->n ||
-            g_batch.dA[i] != dA[i] || g_batch.M[i] != M[i])
+    for (int i = 0; i < count; i++) {
+        if (B->plans[i] != plans[i] || B->serial[i] != plans[i]->serial || B->n[i] != plans[i]->n ||
+            B->M[i] != M[i])
             return 0;
+        if (B->dA[i] != dA[i]) *same = 0;
+    }
     return 1;
 }
 
-static int batch_cache_store(ft_schedule *S, const ft_rotation_plan *const *plans, int kind, int direction,
+/* A cached band-systolic schedule on other matrices, in `stream`'s order. */
+static int batch_cache_rebase(ft_batch_cache *B, int precision, void *const *dA, int count, void *stream) {
+    ft_schedule *S = B->sched;
+    const long long esz = precision == 0 ? sizeof(double) : sizeof(float);
+    long long *off = malloc(sizeof(*off) * (size_t)count);
+    if (!off) return FTAMD_ENOMEM;
+    int rc = ftamd_hip_event_wait(B->event, stream);
+    for (int i = 0; i < count; i++) off[i] = ftamd_sys_matrix_offset(dA, i, esz);
+    if (rc == FTAMD_OK)
+        rc = ftamd_hip_sys_rebase((FtamdSysChain *)S->sys_launch.chains, S->d_mat, S->sys_launch.nchains, off, count,
+                                  stream);
+    free(off);
+    if (rc != FTAMD_OK) return rc;
+    S->sys_launch.A = dA[0];
+    for (int i = 0; i < count; i++) B->dA[i] = dA[i];
+    return FTAMD_OK;
+}
+
+static int batch_cache_store(ft_batch_cache *B, ft_schedule *S, const ft_rotation_plan *const *plans, int kind, int direction,
                              int precision, void *const *dA, const int *M, int count, int L, int W, int engine,
                              int part) {
     size_t c = (size_t)count;
-    g_batch.plans = malloc(sizeof(*g_batch.plans) * c);
-    g_batch.serial = malloc(sizeof(*g_batch.serial) * c);
-    g_batch.n = malloc(sizeof(int) * c);
-    g_batch.dA = malloc(sizeof(void *) * c);
-    g_batch.M = malloc(sizeof(int) * c);
-    if (!g_batch.plans || !g_batch.serial || !g_batch.n || !g_batch.dA || !g_batch.M) {
-        g_batch.sched = S;
-        batch_cache_clear_locked();
+    B->plans = malloc(sizeof(*B->plans) * c);
+    B->serial = malloc(sizeof(*B->serial) * c);
+    B->n = malloc(sizeof(int) * c);
+    B->dA = malloc(sizeof(void *) * c);
+    B->M = malloc(sizeof(int) * c);
+    if (!B->plans || !B->serial || !B->n || !B->dA || !B->M) {
+        B->sched = S;
+        batch_cache_clear_locked(B);
         return FTAMD_ENOMEM;
     }
     for (int i = 0; i < count; i++) {
-        g_batch.plans[i] = plans[i];
-        g_batch.serial[i] = plans[i]->serial;
-        g_batch.n[i] = plans[i]->n;
-        g_batch.dA[i] = dA[i];
-        g_batch.M[i] = M[i];
+        B->plans[i] = plans[i];
+        B->serial[i] = plans[i]->serial;
+        B->n[i] = plans[i]->n;
+        B->dA[i] = dA[i];
+        B->M[i] = M[i];
     }
-    g_batch.sched = S;
-    g_batch.count = count;
-    g_batch.kind = kind;
-    g_batch.dir = direction;
-    g_batch.precision = precision;
-    g_batch.L = L;
-    g_batch.W = W;
-    g_batch.part = part;
-    g_batch.engine = engine;
+    B->sched = S;
+    B->count = count;
+    B->kind = kind;
+    B->dir = direction;
+    B->precision = precision;
+    B->L = L;
+    B->W = W;
+    B->part = part;
+    B->engine = engine;
     return FTAMD_OK;
 }
 /* Validates a batch and uploads the largest plan's table; *big gets that plan. */
@@ -1803,10 +1851,11 @@ static int batch_build_sys(const ft_rotation_plan *const *plans, int kind, int l
     }
     FtamdSysBand *bands = NULL;
     FtamdSysChain *ch = NULL;
-    int nb = 0, nch = 0, nprog = 0;
+    int nb = 0, nch = 0, nprog = 0, *mat = NULL;
     const void *tab_base = NULL;
     if (rc == FTAMD_OK)
-        rc = ftamd_sys_batch(plans, tabs, dA, M, count, layout, maxpart, &bands, &nb, &ch, &nch, &nprog, &tab_base);
+        rc = ftamd_sys_batch(plans, tabs, dA, M, count, layout, maxpart, &bands, &nb, &ch, &nch, &nprog, &mat,
+                             &tab_base);
     free(tabs);
     if (rc != FTAMD_OK) {
         free(bands);
@@ -1815,9 +1864,18 @@ static int batch_build_sys(const ft_rotation_plan *const *plans, int kind, int l
     }
     ft_schedule *S = calloc(1, sizeof(ft_schedule));
     if (!S) rc = FTAMD_ENOMEM;
+    /* the bands, then each chain's transform */
+    const size_t nbytes = sizeof(FtamdSysBand) * (size_t)nb, mbytes = sizeof(int) * (size_t)nch;
+    char *extra = rc == FTAMD_OK ? malloc(nbytes + mbytes + 1) : NULL;
+    if (rc == FTAMD_OK && !extra) rc = FTAMD_ENOMEM;
     void *dbands = NULL;
-    if (rc == FTAMD_OK)
-        rc = sys_upload(S, ch, nch, nprog, bands, bands, sizeof(FtamdSysBand) * (size_t)nb, &dbands);
+    if (rc == FTAMD_OK) {
+        memcpy(extra, bands, nbytes);
+        if (nch > 0) memcpy(extra + nbytes, mat, mbytes);
+        rc = sys_upload(S, ch, nch, nprog, bands, extra, nbytes + mbytes, &dbands);
+    }
+    free(extra);
+    free(mat);
     free(bands);
     free(ch);
     if (rc != FTAMD_OK) {
@@ -1835,6 +1893,7 @@ static int batch_build_sys(const ft_rotation_plan *const *plans, int kind, int l
     a->rowmask = sys_rowmask(kind, layout);
     a->tab = tab_base;
     a->A = dA[0];
+    S->d_mat = (const int *)((const char *)dbands + nbytes);
     *out = S;
     return FTAMD_OK;
 }
@@ -1902,23 +1961,48 @@ int ft_gpu_execute_batch(const ft_rotation_plan *const *plans, int kind, int dir
     ftamd_choose(geo, precision, direction, 1, big->n, &ch);
     /* the cache key holds every choice the schedule was built with */
     const int L = ch.L, W = ch.W, engine = ch.engine * 2 + ch.forced, part = ch.maxpart * 16 + ch.wg_per_cu;
-    pthread_mutex_lock(&g_batch.lock);
-    ft_schedule *S = g_batch.sched;
-    if (!batch_cache_hit(plans, kind, direction, precision, dA, M, count, L, W, engine, part)) {
-        batch_cache_clear_locked();
-        S = NULL;
-        rc = batch_build(plans, geo, layout, direction, precision, dA, M, count, big, &ch, &S);
-        if (rc == FTAMD_OK)
-            rc = batch_cache_store(S, plans, kind, direction, precision, dA, M, count, L, W, engine, part);
+    pthread_mutex_lock(&g_batch_lock);
+    const int capturing = ftamd_hip_capturing(stream);
+    /* a schedule of these matrices, else one of other matrices, else the least
+     * recently used entry (an empty one first) */
+    ft_batch_cache *B = NULL, *other = NULL, *old = &g_batches[0];
+    for (int k = 0; k < FTAMD_BATCHES && !B; k++) {
+        ft_batch_cache *E = &g_batches[k];
+        int same = 0;
+        if (batch_cache_hit(E, plans, kind, direction, precision, dA, M, count, L, W, engine, part, &same)) {
+            if (same) B = E;
+            else other = E;
+        }
+        if (old->sched && (!E->sched || E->used < old->used)) old = E;
+    }
+    if (!B && other && other->sched->sys && !other->captured && !capturing) {
+        B = other;
+        rc = batch_cache_rebase(B, precision, dA, count, stream);
         if (rc != FTAMD_OK) {
-            pthread_mutex_unlock(&g_batch.lock);
+            batch_cache_clear_locked(B);
+            pthread_mutex_unlock(&g_batch_lock);
             return rc;
         }
     }
+    if (!B) {
+        B = other ? other : old;
+        batch_cache_clear_locked(B);
+        ft_schedule *N = NULL;
+        rc = batch_build(plans, geo, layout, direction, precision, dA, M, count, big, &ch, &N);
+        if (rc == FTAMD_OK)
+            rc = batch_cache_store(B, N, plans, kind, direction, precision, dA, M, count, L, W, engine, part);
+        if (rc != FTAMD_OK) {
+            pthread_mutex_unlock(&g_batch_lock);
+            return rc;
+        }
+    }
+    ft_schedule *S = B->sched;
+    B->used = ++g_batch_calls;
     t_last_engine = S->sys ? FT_GPU_ENGINE_SYSTOLIC : FT_GPU_ENGINE_PIPELINE;
     rc = launch(S, precision, geo, direction, NULL, stream);
+    if (capturing || (S->sys && ftamd_hip_event_record(&B->event, stream) != FTAMD_OK)) B->captured = 1;
     if (rc == FTAMD_OK) pending_add(S, stream);
-    pthread_mutex_unlock(&g_batch.lock);
+    pthread_mutex_unlock(&g_batch_lock);
     return rc;
 }
 

@@ -163,6 +163,18 @@ typedef struct {
 } FtamdSysLaunch;
 
 int ftamd_hip_sys_launch(const FtamdSysLaunch *a, int precision, int S, void *stream);
+/* New matrices for the chains of a batch (device arrays): chain c belongs to
+ * matrix mat[c], whose offset (elements from the launch's A) becomes
+ * off[mat[c]] (host array, passed by value). */
+int ftamd_hip_sys_rebase(FtamdSysChain *chains, const int *mat, int nchains, const long long *off, int count,
+                         void *stream);
+/* Whether `stream` is being captured (or cannot be asked). */
+int ftamd_hip_capturing(void *stream);
+/* An event (made on first use) after the work of `stream` so far; `stream`
+ * waits for it. */
+int ftamd_hip_event_record(void **event, void *stream);
+int ftamd_hip_event_wait(void *event, void *stream);
+void ftamd_hip_event_destroy(void *event);
 
 /* Triangular products of the harmonic transforms (drivers.c:833-1021), out
  * of place from X (n x M, column-major) into Y (same shape, another buffer).

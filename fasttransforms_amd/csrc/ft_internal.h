@@ -35,6 +35,8 @@ typedef struct ft_schedule {
     int wg_per_cu;     /* pipelined: workgroups per CU it was built for, 0: no cap */
     FtamdSysLaunch sys_launch;
     void *d_sys;
+    /* a band-systolic batch: the matrix of each chain (device) */
+    const int *d_mat;
     double flops;            /* algorithmic flops (6 per rotation) */
 } ft_schedule;
 
@@ -155,9 +157,10 @@ int ftamd_sys_chains_spin(const ft_rotation_plan *RP, const ft_sys_tables *T, in
 int ftamd_sys_debug_tet(const ft_rotation_plan *RP, int dir, int S, int part, int N, int L, int m0, int count,
                         int maxpart, FtamdSysBand **bands, int *nbands, double **tab, long long *nentries,
                         FtamdSysChain **chains, int *nchains);
+long long ftamd_sys_matrix_offset(void *const *dA, int i, long long esz);
 int ftamd_sys_batch(const ft_rotation_plan *const *plans, ft_sys_tables *const *tabs, void *const *dA,
                     const int *M, int count, int layout, int maxpart, FtamdSysBand **bands, int *nbands,
                     FtamdSysChain **chains,
-                    int *nchains, int *nprog, const void **tab_base);
+                    int *nchains, int *nprog, int **mat, const void **tab_base);
 
 #endif /* FT_INTERNAL_H */

@@ -25,3 +25,36 @@ extern "C" int ftamd_hip_sys_launch(const FtamdSysLaunch *a, int precision, int 
     if (e == hipSuccess) return FTAMD_OK;
     return e == hipErrorOutOfMemory ? FTAMD_ENOMEM : FTAMD_EDEVICE;
 }
+
+namespace ftsys {
+
+// The offsets of a batch's matrices (elements from the launch's A), passed by value.
+struct Bases {
+    long long off[256];
+    int m0, count;
+};
+
+// Chains of the matrices m0 .. m0 + count - 1 take their matrix's offset.
+__global__ void __launch_bounds__(256) rebase_kernel(FtamdSysChain *chains, const int *mat, int nchains, Bases b) {
+    const int c = blockIdx.x * 256 + threadIdx.x;
+    if (c >= nchains) return;
+    const int m = mat[c] - b.m0;
+    if (m >= 0 && m < b.count) chains[c].aoff = b.off[m];
+}
+
+}  // namespace ftsys
+
+extern "C" int ftamd_hip_sys_rebase(FtamdSysChain *chains, const int *mat, int nchains, const long long *off,
+                                    int count, void *stream) {
+    if (nchains <= 0) return FTAMD_OK;
+    for (int m0 = 0; m0 < count; m0 += 256) {
+        ftsys::Bases b;
+        b.m0 = m0;
+        b.count = count - m0 < 256 ? count - m0 : 256;
+        for (int k = 0; k < 256; ++k) b.off[k] = k < b.count ? off[m0 + k] : 0;
+        hipLaunchKernelGGL(ftsys::rebase_kernel, dim3((nchains + 255) / 256), dim3(256), 0, (hipStream_t)stream,
+                           chains, mat, nchains, b);
+    }
+    hipError_t e = hipGetLastError();
+    return e == hipSuccess ? FTAMD_OK : FTAMD_EDEVICE;
+}

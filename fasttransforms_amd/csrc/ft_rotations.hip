@@ -169,6 +169,31 @@ int ftamd_hip_d2d(void *dst, const void *src, size_t bytes, void *stream) {
 
 int ftamd_hip_device_sync(void) { return map_err(hipDeviceSynchronize()); }
 
+int ftamd_hip_capturing(void *stream) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing((hipStream_t)stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return 1;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
+int ftamd_hip_event_record(void **event, void *stream) {
+    if (!*event && hipEventCreateWithFlags((hipEvent_t *)event, hipEventDisableTiming) != hipSuccess) {
+        *event = nullptr;
+        return map_err(hipGetLastError());
+    }
+    return map_err(hipEventRecord((hipEvent_t)*event, (hipStream_t)stream));
+}
+
+int ftamd_hip_event_wait(void *event, void *stream) {
+    return map_err(hipStreamWaitEvent((hipStream_t)stream, (hipEvent_t)event, 0));
+}
+
+void ftamd_hip_event_destroy(void *event) {
+    if (event) (void)hipEventDestroy((hipEvent_t)event);
+}
+
 int ftamd_hip_sync(void *stream) { return map_err(hipStreamSynchronize((hipStream_t)stream)); }
 
 int ftamd_hip_last_runtime_error(void) { return g_hip_err; }

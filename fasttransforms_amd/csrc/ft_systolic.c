@@ -659,16 +659,24 @@ int ftamd_sys_chains_tet(const ft_rotation_plan *RP, const ft_sys_tables *T, int
     return FTAMD_OK;
 }
 
+/* Elements (of esz bytes) from a batch's first matrix to matrix i. */
+long long ftamd_sys_matrix_offset(void *const *dA, int i, long long esz) {
+    return ((long long)(uintptr_t)dA[i] - (long long)(uintptr_t)dA[0]) / esz;
+}
+
 /* Bands and chains of a batch of transforms of one kind, direction,
  * precision and S (every plan's tables built): the bands of each distinct
  * plan once, their table offsets taken from the first plan's tables, the
  * chains of every transform with its bands, matrix offset from dA[0] and
- * column stride, longest first.  FTAMD_EINVAL if a chain does not fit. */
+ * column stride, longest first, and the transform of each (*mat_out).
+ * FTAMD_EINVAL if a chain does not fit. */
 int ftamd_sys_batch(const ft_rotation_plan *const *plans, ft_sys_tables *const *tabs, void *const *dA,
                     const int *M, int count, int layout, int maxpart, FtamdSysBand **bands_out, int *nbands_out,
-                    FtamdSysChain **chains_out, int *nchains_out, int *nprog_out, const void **tab_base) {
+                    FtamdSysChain **chains_out, int *nchains_out, int *nprog_out, int **mat_out,
+                    const void **tab_base) {
     *bands_out = NULL;
     *chains_out = NULL;
+    *mat_out = NULL;
     *nbands_out = *nchains_out = *nprog_out = 0;
     *tab_base = count > 0 ? tabs[0]->d_tab : NULL;
     if (count <= 0) return FTAMD_OK;
@@ -713,7 +721,7 @@ int ftamd_sys_batch(const ft_rotation_plan *const *plans, ft_sys_tables *const *
         }
         for (int c = 0; rc == FTAMD_OK && c < nch; c++) {
             ch[c].band0 += first[k];
-            ch[c].aoff = ((long long)(uintptr_t)dA[i] - (long long)(uintptr_t)dA[0]) / esz;
+            ch[c].aoff = i; /* its transform, until the chains are in order */
             all[nall++] = ch[c];
         }
         free(ch);
@@ -728,11 +736,18 @@ int ftamd_sys_batch(const ft_rotation_plan *const *plans, ft_sys_tables *const *
     sort_chains(all, nall);
     int nparts = 0, nprog = 0;
     rc = all ? split_alloc(&all, nall, maxpart, &nparts, &nprog) : FTAMD_OK;
+    int *mat = rc == FTAMD_OK ? malloc(sizeof(int) * (size_t)(nparts > 0 ? nparts : 1)) : NULL;
+    if (rc == FTAMD_OK && !mat) rc = FTAMD_ENOMEM;
     if (rc != FTAMD_OK) {
         free(bands);
         free(all);
         return rc;
     }
+    for (int c = 0; c < nparts; c++) {
+        mat[c] = (int)all[c].aoff;
+        all[c].aoff = ftamd_sys_matrix_offset(dA, mat[c], esz);
+    }
+    *mat_out = mat;
     *bands_out = bands;
     *nbands_out = nb;
     *chains_out = all;
