@@ -163,6 +163,20 @@ typedef struct {
 } FtamdSysLaunch;
 
 int ftamd_hip_sys_launch(const FtamdSysLaunch *a, int precision, int S, void *stream);
+/* The classes of a plan's sequences, for its tables: sequence k of class c is
+ * j = jtop - jstep*k, its class row e matrix row rstep*e + rpar; its bands are
+ * band0 .. band0+nb-1. */
+typedef struct {
+    int kind, n, dir, ncls;
+    struct {
+        int jtop, jstep, K, rpar, rstep, band0, nb;
+    } cls[4];
+} FtamdSysClasses;
+/* Every band's table from the plan's sines and cosines (device arrays):
+ * tab[b.tab ..] of each band b, FP64 (precision 0) or rounded to FP32.  S:
+ * sequences a lane; nbands <= 65535, maxsteps the most steps of a band. */
+int ftamd_hip_sys_tables(void *tab, int precision, int S, const FtamdSysClasses *c, const FtamdSysBand *bands,
+                         int nbands, int maxsteps, const double *sn, const double *cs, void *stream);
 /* New matrices for the chains of a batch (device arrays): chain c belongs to
  * matrix mat[c], whose offset (elements from the launch's A) becomes
  * off[mat[c]] (host array, passed by value). */

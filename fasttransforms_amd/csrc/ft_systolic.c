@@ -108,11 +108,10 @@ int ftamd_sys_choose_S(int kind, int n, int precision) {
     return 0;
 }
 
-/* Bands of every class and their tables, on the host (T->bands, *host). */
-static int tables_host(const ft_rotation_plan *RP, int dir, int precision, int S, ft_sys_tables *T, void **host,
-                       long long *nentries) {
+/* Bands of every class (T->bands) and the entries of all their tables. */
+static int tables_bands(const ft_rotation_plan *RP, int dir, int precision, int S, ft_sys_tables *T,
+                        long long *nentries) {
     const int kind = RP->kind, n = RP->n, B = FTAMD_SYS_LANES * S, U = FTAMD_SYS_UNROLL, PF = FTAMD_SYS_PREFETCH;
-    *host = NULL;
     T->S = S;
     T->dir = dir;
     T->precision = precision;
@@ -142,8 +141,19 @@ static int tables_host(const ft_rotation_plan *RP, int dir, int precision, int S
             entries += (long long)(bd->steps + PF) * FTAMD_SYS_LANES * S;
         }
     }
-    size_t esz = precision == 0 ? sizeof(double) : sizeof(float);
-    void *h = malloc((size_t)(entries > 0 ? entries : 1) * 2 * esz);
+    *nentries = entries;
+    return FTAMD_OK;
+}
+
+/* Bands and tables on the host, in FP64 (diagnostics; ftamd_sys_tables_build
+ * has the device make the tables). */
+static int tables_host(const ft_rotation_plan *RP, int dir, int S, ft_sys_tables *T, double **host,
+                       long long *nentries) {
+    const int kind = RP->kind, n = RP->n, B = FTAMD_SYS_LANES * S, PF = FTAMD_SYS_PREFETCH;
+    *host = NULL;
+    const int rc = tables_bands(RP, dir, 0, S, T, nentries);
+    if (rc != FTAMD_OK) return rc;
+    double *h = malloc((size_t)(*nentries > 0 ? *nentries : 1) * 2 * sizeof(double));
     if (!h) return FTAMD_ENOMEM;
     for (int c = 0; c < T->ncls; c++) {
         const sys_class *cl = &T->cls[c];
@@ -154,8 +164,7 @@ static int tables_host(const ft_rotation_plan *RP, int dir, int precision, int S
                     /* lane i holds sequences q = S*i .. S*i+S-1: entry (t, i, s),
                      * stored slot-major in FP64 */
                     int i_lane = q / S, s_slot = q % S;
-                    long long at = bd->tab + (long long)t * B +
-                                   (FTAMD_SYS_SLOT_MAJOR(precision) ? s_slot * FTAMD_SYS_LANES + i_lane : q);
+                    long long at = bd->tab + (long long)t * B + s_slot * FTAMD_SYS_LANES + i_lane;
                     double sv = 0.0, cv = 1.0;
                     if (q < bd->nseq) {
                         int g = bd->gbase + q;
@@ -170,18 +179,12 @@ static int tables_host(const ft_rotation_plan *RP, int dir, int precision, int S
                             cv = RP->c[ix];
                         }
                     }
-                    if (precision == 0) {
-                        ((double *)h)[2 * at] = sv;
-                        ((double *)h)[2 * at + 1] = cv;
-                    } else {
-                        ((float *)h)[2 * at] = (float)sv;
-                        ((float *)h)[2 * at + 1] = (float)cv;
-                    }
+                    h[2 * at] = sv;
+                    h[2 * at + 1] = cv;
                 }
         }
     }
     *host = h;
-    *nentries = entries;
     return FTAMD_OK;
 }
 
@@ -189,21 +192,45 @@ int ftamd_sys_tables_build(const ft_rotation_plan *RP, int dir, int precision, i
     *out = NULL;
     ft_sys_tables *T = calloc(1, sizeof(ft_sys_tables));
     if (!T) return FTAMD_ENOMEM;
-    void *host = NULL;
     long long entries = 0;
-    int rc = tables_host(RP, dir, precision, S, T, &host, &entries);
+    int rc = tables_bands(RP, dir, precision, S, T, &entries);
     size_t esz = precision == 0 ? sizeof(double) : sizeof(float);
     T->tab_bytes = (size_t)entries * 2 * esz;
-    /* the kernel addresses the tables with 32-bit byte offsets */
     if (rc == FTAMD_OK && T->tab_bytes >= 0x7fffffffULL) rc = FTAMD_EINVAL;
     if (rc == FTAMD_OK) rc = ftamd_hip_malloc(&T->d_tab, (size_t)(entries > 0 ? entries : 1) * 2 * esz);
     if (rc == FTAMD_OK)
         rc = ftamd_hip_malloc(&T->d_bands, sizeof(FtamdSysBand) * (size_t)(T->nbands > 0 ? T->nbands : 1));
-    if (rc == FTAMD_OK && entries > 0) rc = ftamd_hip_h2d(T->d_tab, host, (size_t)entries * 2 * esz, NULL);
-    if (rc == FTAMD_OK && T->nbands > 0)
+    if (rc == FTAMD_OK && T->nbands > 0) {
+        const size_t bytes = sizeof(double) * (size_t)RP->nsc;
+        FtamdSysClasses c;
+        memset(&c, 0, sizeof(c));
+        c.kind = RP->kind;
+        c.n = RP->n;
+        c.dir = dir;
+        c.ncls = T->ncls;
+        int maxsteps = 0;
+        for (int k = 0; k < T->ncls; k++) {
+            c.cls[k].jtop = T->cls[k].jtop;
+            c.cls[k].jstep = T->cls[k].jstep;
+            c.cls[k].K = T->cls[k].K;
+            c.cls[k].rpar = T->cls[k].rpar;
+            c.cls[k].rstep = T->cls[k].rstep;
+            c.cls[k].band0 = T->band0[k];
+            c.cls[k].nb = T->nb[k];
+        }
+        for (int b = 0; b < T->nbands; b++)
+            if (T->bands[b].steps > maxsteps) maxsteps = T->bands[b].steps;
+        char *sc = NULL; /* the plan's sines, then its cosines */
         rc = ftamd_hip_h2d(T->d_bands, T->bands, sizeof(FtamdSysBand) * (size_t)T->nbands, NULL);
-    if (rc == FTAMD_OK) rc = ftamd_hip_sync(NULL);
-    free(host);
+        if (rc == FTAMD_OK) rc = ftamd_hip_malloc((void **)&sc, 2 * bytes);
+        if (rc == FTAMD_OK) rc = ftamd_hip_h2d(sc, RP->s, bytes, NULL);
+        if (rc == FTAMD_OK) rc = ftamd_hip_h2d(sc + bytes, RP->c, bytes, NULL);
+        if (rc == FTAMD_OK)
+            rc = ftamd_hip_sys_tables(T->d_tab, precision, S, &c, (const FtamdSysBand *)T->d_bands, T->nbands, maxsteps,
+                                      (const double *)sc, (const double *)(sc + bytes), NULL);
+        if (rc == FTAMD_OK) rc = ftamd_hip_sync(NULL);
+        ftamd_hip_free(sc);
+    }
     if (rc != FTAMD_OK) {
         ftamd_sys_tables_free(T);
         return rc;
@@ -763,8 +790,8 @@ int ftamd_sys_debug_spin(const ft_rotation_plan *RP, int dir, int S, int s, int 
                          int *nbands, double **tab, long long *nentries, FtamdSysChain **chains, int *nchains) {
     ft_sys_tables T;
     memset(&T, 0, sizeof(T));
-    void *host = NULL;
-    int rc = tables_host(RP, dir, 0, S, &T, &host, nentries);
+    double *host = NULL;
+    int rc = tables_host(RP, dir, S, &T, &host, nentries);
     int nprog = 0;
     if (rc == FTAMD_OK) rc = ftamd_sys_chains_spin(RP, &T, s, M, maxpart, chains, nchains, &nprog);
     if (rc != FTAMD_OK) {
@@ -786,8 +813,8 @@ int ftamd_sys_debug_tet(const ft_rotation_plan *RP, int dir, int S, int part, in
                         FtamdSysChain **chains, int *nchains) {
     ft_sys_tables T;
     memset(&T, 0, sizeof(T));
-    void *host = NULL;
-    int rc = tables_host(RP, dir, 0, S, &T, &host, nentries);
+    double *host = NULL;
+    int rc = tables_host(RP, dir, S, &T, &host, nentries);
     int nprog = 0;
     if (rc == FTAMD_OK) rc = ftamd_sys_chains_tet(RP, &T, part, N, L, m0, count, maxpart, chains, nchains, &nprog);
     if (rc != FTAMD_OK) {
@@ -809,8 +836,8 @@ int ftamd_sys_debug_host(const ft_rotation_plan *RP, int dir, int S, int M, int 
                          int *nchains) {
     ft_sys_tables T;
     memset(&T, 0, sizeof(T));
-    void *host = NULL;
-    int rc = tables_host(RP, dir, 0, S, &T, &host, nentries);
+    double *host = NULL;
+    int rc = tables_host(RP, dir, S, &T, &host, nentries);
     int nprog = 0;
     if (rc == FTAMD_OK) rc = ftamd_sys_chains(RP, &T, M, layout, maxpart, chains, nchains, &nprog);
     if (rc != FTAMD_OK) {
