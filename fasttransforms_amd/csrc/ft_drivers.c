@@ -1898,10 +1898,10 @@ static int batch_build_sys(const ft_rotation_plan *const *plans, int kind, int l
     return FTAMD_OK;
 }
 
-/* Builds the schedule of a validated batch: the pipelined engine, or the
- * band-systolic one when forced (it keeps one chain per CU, and the many
- * short chains of a batch of small transforms leave most of each CU idle:
- * 20.2 ms against 10.4 ms for 512 sph transforms of degree 32..1018). */
+/* Builds the schedule of a validated batch on the engine the tuning table
+ * (or the caller) names.  256 sph transforms of degree 32 .. 1024 hi2lo in
+ * FP64 take 3.8 ms band-systolic and 4.4 ms pipelined, disk ones 14.3 and 12.7
+ * (long chains in several parts). */
 static int batch_build(const ft_rotation_plan *const *plans, int kind, int layout, int direction, int precision,
                        void *const *dA, const int *M, int count, ft_rotation_plan *big, const ftamd_choice *ch,
                        ft_schedule **out) {

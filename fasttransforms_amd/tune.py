@@ -28,7 +28,7 @@ import numpy as np
 import fasttransforms_amd as ft
 
 KINDS = {"sph": (ft.SPH, ()), "tri": (ft.TRI, (0.0, 0.0, 0.0)), "disk": (ft.DISK, (0.0, 0.0))}
-SIZES = [64, 128, 256, 512, 1024, 2048]
+SIZES = [64, 128, 256, 512, 768, 1024, 1448, 2048]
 QUICK_SIZES = [256, 1024]
 BATCH_NMAX = [256, 1024]
 SYS_PARTS = [16, 12, 8]
