@@ -104,7 +104,7 @@ typedef struct {
 typedef struct {
     long long tab;    /* entry offset of the band's table: [steps + PREFETCH] steps of LANES*S (s, c) pairs */
     int R;            /* the band's row stream is rows 0 .. R of the class */
-    int steps;        /* steps the band runs: R + (S+1)*(LANES-1) + S + 1 rounded up to UNROLL */
+    int steps;        /* R + (S+1)*(LANES-1) + S + 1 rounded up to UNROLL (it may run a block more, on identities) */
     int gbase;        /* position of the band's first sequence in the class, in application order */
     int nseq;         /* sequences of the class in the band (the rest are identities) */
 } FtamdSysBand;

@@ -291,8 +291,8 @@ int ft_gpu_execute_tet(const ft_rotation_plan *RP1, const ft_rotation_plan *RP2,
  * the bivariate Fourier series sph2fourier produces -> values on the
  * N x M grid theta_i = (i+1/2) pi / N, phi_j = 2 pi j / M) and analysis (the
  * inverse) on the sphere, and their vector-field variants, on the GPU
- * (hipFFT plus this library's kernels in place of FFTW).  The plan holds
- * device work buffers (about 24 N M bytes); flags are ignored.  X is N x M
+ * (this library's kernels in place of FFTW; hipFFT for lines longer than 4096).
+ * The plan holds device work buffers (about 8 N M bytes); flags are ignored.  X is N x M
  * column-major, host or device, M odd, overwritten in place.  Synthesis 'N'
  * and analysis 'T' take a synthesis plan, synthesis 'T' and analysis 'N' an
  * analysis plan (as the reference's own tests pair them); another plan, or
@@ -480,9 +480,9 @@ int ft_gpu_synchronize(void *stream);
 /* Batched transforms of uneven degree in one launch.  plans[i] may differ in
  * n (plans of one constructor and one set of parameters); dA[i] is
  * plans[i]->n x M[i] on the device.
- * Every transform runs as one persistent, cost-ordered launch.  The schedule
- * of the last argument list is cached; a call with another list replaces it,
- * so a HIP graph that captured this call is valid only until then (use a
+ * Every transform runs as one persistent, cost-ordered launch.  The schedules
+ * of the last eight argument lists are cached; calls with other lists replace
+ * them, so a HIP graph that captured this call is valid only until then (use a
  * batch plan below for graphs). */
 int ft_gpu_execute_batch(const ft_rotation_plan *const *plans, int kind, int direction, int precision,
                          void *const *dA, const int *M, int count, void *stream);
