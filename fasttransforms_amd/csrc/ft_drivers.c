@@ -102,6 +102,8 @@ void ftamd_choose(int kind, int precision, int dir, int batch, int n, ftamd_choi
      * CU (512 sph transforms of degree 32..1018: 9.9 ms capped, 10.4 ms not) */
     c->forced = ke != FT_GPU_ENGINE_AUTO;
     c->engine = c->forced ? ke : found ? te : (batch ? FT_GPU_ENGINE_PIPELINE : FT_GPU_ENGINE_SYSTOLIC);
+    if (!c->forced && c->engine == FT_GPU_ENGINE_SYSTOLIC && !ftamd_sys_applies(kind, n, dir, precision))
+        c->engine = FT_GPU_ENGINE_PIPELINE;
     c->maxpart = km ? km : (found && tm) ? tm : FTAMD_SYS_WAVES;
     c->L = kL ? kL : (found && tL) ? tL : 4;
     c->W = kW ? kW : (found && tW) ? tW : 16;

@@ -96,7 +96,8 @@ void ftamd_batch_forget_plan(const ft_rotation_plan *RP);
 int ftamd_engine(void);
 
 /* The engine and shape a launch uses: the knobs (ft_gpu_set_*) where set,
- * else the autotuning table's row, else the built-in choice. */
+ * else the autotuning table's row, else the built-in choice; the pipelined
+ * engine where the band-systolic one does not run the degree (unless forced). */
 typedef struct {
     int engine;     /* FT_GPU_ENGINE_PIPELINE or FT_GPU_ENGINE_SYSTOLIC (preferred; forced if the knob is) */
     int forced;     /* the engine knob is set */
@@ -133,6 +134,7 @@ int ftamd_spin_upload(ft_spin_rotation_plan *P);
 
 /* ft_systolic.c */
 int ftamd_sys_choose_S(int kind, int n, int precision);
+int ftamd_sys_applies(int kind, int n, int dir, int precision);
 int ftamd_sys_tables_build(const ft_rotation_plan *RP, int dir, int precision, int S, ft_sys_tables **out);
 void ftamd_sys_tables_free(ft_sys_tables *T);
 int ftamd_sys_tables_S(const ft_sys_tables *T);

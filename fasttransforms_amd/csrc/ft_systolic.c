@@ -82,7 +82,6 @@ struct ft_sys_tables {
     int nbands;
     void *d_bands;
     void *d_tab;
-    size_t tab_bytes;
 };
 
 int ftamd_sys_tables_S(const ft_sys_tables *T) { return T->S; }
@@ -108,10 +107,55 @@ int ftamd_sys_choose_S(int kind, int n, int precision) {
     return 0;
 }
 
+/* Band b of a class; tab (its table's place) stays 0. */
+static FtamdSysBand band_of(int kind, int n, const sys_class *cl, int dir, int S, int b) {
+    const int B = FTAMD_SYS_LANES * S, g0 = B * b, nseq = cl->K - g0 < B ? cl->K - g0 : B;
+    /* the stream's top row: one above the longest sequence's top */
+    const int klong = dir == 0 ? g0 + nseq - 1 : cl->K - 1 - g0;
+    FtamdSysBand bd;
+    memset(&bd, 0, sizeof(bd));
+    bd.R = class_top(kind, n, cl, cl->jtop - cl->jstep * klong) + 1;
+    if (bd.R < 0) bd.R = 0;
+    /* the last sequence emits position R at step R + delay + 1 */
+    bd.steps = round_up(bd.R + sys_delay(S, B - 1) + 2, FTAMD_SYS_UNROLL);
+    bd.gbase = g0;
+    bd.nseq = nseq;
+    return bd;
+}
+
+static int class_bands(const sys_class *cl, int S) {
+    const int B = FTAMD_SYS_LANES * S;
+    return (cl->K + B - 1) / B;
+}
+
+/* (s, c) entries of a band's table */
+static long long band_entries(const FtamdSysBand *bd, int S) {
+    return (long long)(bd->steps + FTAMD_SYS_PREFETCH) * FTAMD_SYS_LANES * S;
+}
+
+/* Whether the band-systolic engine runs a degree: tables below 2 GiB a
+ * direction (FP64 sph n < 16196, tri 16290, disk 11491; FP32 sph n < 22980).
+ * Nothing above that has been run: a launch there takes half a second, about
+ * what a wait's polls last, so those degrees are the pipelined engine's. */
+int ftamd_sys_applies(int kind, int n, int dir, int precision) {
+    const int S = ftamd_sys_choose_S(kind, n, precision);
+    if (S == 0) return 0;
+    if (n <= 4096) return 1; /* at most 0.3 GiB */
+    sys_class cl[4];
+    const int ncls = make_classes(kind, n, cl);
+    long long entries = 0;
+    for (int c = 0; c < ncls; c++)
+        for (int b = 0; b < class_bands(&cl[c], S); b++) {
+            const FtamdSysBand bd = band_of(kind, n, &cl[c], dir, S, b);
+            entries += band_entries(&bd, S);
+        }
+    return entries * 2 * (long long)(precision == 0 ? sizeof(double) : sizeof(float)) < 0x7fffffffLL;
+}
+
 /* Bands of every class (T->bands) and the entries of all their tables. */
 static int tables_bands(const ft_rotation_plan *RP, int dir, int precision, int S, ft_sys_tables *T,
                         long long *nentries) {
-    const int kind = RP->kind, n = RP->n, B = FTAMD_SYS_LANES * S, U = FTAMD_SYS_UNROLL, PF = FTAMD_SYS_PREFETCH;
+    const int kind = RP->kind, n = RP->n;
     T->S = S;
     T->dir = dir;
     T->precision = precision;
@@ -119,28 +163,18 @@ static int tables_bands(const ft_rotation_plan *RP, int dir, int precision, int 
     long long entries = 0;
     for (int c = 0; c < T->ncls; c++) {
         T->band0[c] = T->nbands;
-        T->nb[c] = (T->cls[c].K + B - 1) / B;
+        T->nb[c] = class_bands(&T->cls[c], S);
         T->nbands += T->nb[c];
     }
     T->bands = calloc((size_t)(T->nbands > 0 ? T->nbands : 1), sizeof(FtamdSysBand));
     if (!T->bands) return FTAMD_ENOMEM;
-    for (int c = 0; c < T->ncls; c++) {
-        const sys_class *cl = &T->cls[c];
+    for (int c = 0; c < T->ncls; c++)
         for (int b = 0; b < T->nb[c]; b++) {
             FtamdSysBand *bd = &T->bands[T->band0[c] + b];
-            int g0 = B * b, nseq = cl->K - g0 < B ? cl->K - g0 : B;
-            /* the stream's top row: one above the longest sequence's top */
-            int klong = dir == 0 ? g0 + nseq - 1 : cl->K - 1 - g0;
-            bd->R = class_top(kind, n, cl, cl->jtop - cl->jstep * klong) + 1;
-            if (bd->R < 0) bd->R = 0;
-            /* the last sequence emits position R at step R + delay + 1 */
-            bd->steps = round_up(bd->R + sys_delay(S, B - 1) + 2, U);
-            bd->gbase = g0;
-            bd->nseq = nseq;
+            *bd = band_of(kind, n, &T->cls[c], dir, S, b);
             bd->tab = entries;
-            entries += (long long)(bd->steps + PF) * FTAMD_SYS_LANES * S;
+            entries += band_entries(bd, S);
         }
-    }
     *nentries = entries;
     return FTAMD_OK;
 }
@@ -195,8 +229,7 @@ int ftamd_sys_tables_build(const ft_rotation_plan *RP, int dir, int precision, i
     long long entries = 0;
     int rc = tables_bands(RP, dir, precision, S, T, &entries);
     size_t esz = precision == 0 ? sizeof(double) : sizeof(float);
-    T->tab_bytes = (size_t)entries * 2 * esz;
-    if (rc == FTAMD_OK && T->tab_bytes >= 0x7fffffffULL) rc = FTAMD_EINVAL;
+    if (rc == FTAMD_OK && !ftamd_sys_applies(RP->kind, RP->n, dir, precision)) rc = FTAMD_EINVAL;
     if (rc == FTAMD_OK) rc = ftamd_hip_malloc(&T->d_tab, (size_t)(entries > 0 ? entries : 1) * 2 * esz);
     if (rc == FTAMD_OK)
         rc = ftamd_hip_malloc(&T->d_bands, sizeof(FtamdSysBand) * (size_t)(T->nbands > 0 ? T->nbands : 1));

@@ -88,3 +88,29 @@ def test_slot_assignment(ft, kind, n, maxpart, nxcd, nsx, d):
         work[slot_of[k]] += sum(bands[c.band0 + w].steps for w in range(c.nb))
     biggest = max(sum(bands[c.band0 + w].steps for w in range(c.nb)) for c in chains)
     assert work.max() <= work.mean() + 2 * biggest
+
+
+# the first degree whose band tables reach 2 GiB, from the bands' rows and
+# steps alone: sum over bands of (steps + spare steps) * 32 sequences * 2 values
+BIG = [("sph", 0, 0, 16196), ("sph", 0, 1, 16227), ("tri", 0, 0, 16290), ("tri", 0, 1, 16306), ("disk", 0, 0, 11491),
+       ("sph", 1, 0, 22980)]
+
+
+@pytest.mark.parametrize("kind,precision,direction,n", BIG)
+def test_degrees_past_the_tables(ft, kind, precision, direction, n):
+    """Degrees whose tables the band-systolic engine does not take run on the
+    pipelined engine, whatever the table of choices names, single or batch;
+    only a forced engine is refused (the launch's own answer)."""
+    code = {"sph": ft.SPH, "tri": ft.TRI, "disk": ft.DISK}[kind]
+    nmax = 2 ** 31 - 1
+    try:
+        ft.set_tuning_table([[code, precision, direction, b, 1, nmax, ft.ENGINE_SYSTOLIC, 16, 8, 8, 0] for b in (0, 1)])
+        for batch in (0, 1):
+            assert ft.tuned_choice(kind, precision, direction, batch, n - 1)[0] == ft.ENGINE_SYSTOLIC
+            assert ft.tuned_choice(kind, precision, direction, batch, n) == (ft.ENGINE_PIPELINE, 16, 8, 8, 2 * batch)
+        ft.set_engine(ft.ENGINE_SYSTOLIC)
+        assert ft.tuned_choice(kind, precision, direction, 0, n)[0] == ft.ENGINE_SYSTOLIC
+    finally:
+        ft.set_engine(ft.ENGINE_AUTO)
+        ft.set_tuning_table("compiled")
+    assert ft.tuned_choice(kind, precision, direction, 0, 2 * n)[0] == ft.ENGINE_PIPELINE
