@@ -28,11 +28,15 @@ import numpy as np
 import fasttransforms_amd as ft
 
 KINDS = {"sph": (ft.SPH, ()), "tri": (ft.TRI, (0.0, 0.0, 0.0)), "disk": (ft.DISK, (0.0, 0.0))}
-SIZES = [64, 128, 256, 512, 768, 1024, 1448, 2048]
+# From 1448 on the engines change places: chains get a third and more parts, each
+# of which costs the band-systolic engine (FP64 disk lo2hi n = 1536 1.74 ms against
+# 1.98 pipelined, n = 2400 8.3 against 6.4).
+SIZES = [64, 128, 256, 512, 768, 1024, 1448, 1536, 2048, 2500, 3200, 4000, 5700]
 QUICK_SIZES = [256, 1024]
-BATCH_NMAX = [256, 1024]
+BATCH_NMAX = [256, 1024, 1448, 2048, 2896]
 SYS_PARTS = [16, 12, 8]
 PIPE_SHAPES = [(4, 16), (2, 16), (8, 8), (2, 8)]
+LARGE_SHAPES = [(4, 16), (8, 8)]  # above 2048: two sequences a wave take twice the boundary buffers (disk n = 5792: 110 GB)
 BATCH_SHAPES = [(4, 16, 2), (4, 16, 1), (2, 16, 2), (8, 8, 2)]
 NMAX_INT = 2 ** 31 - 1
 
@@ -135,13 +139,43 @@ def _row(kind, precision, direction, batch, nlo, nhi, cand):
             cand[3] if len(cand) > 3 else 0]
 
 
-def _bands(sizes):
-    """Degree ranges nearest (geometrically) to each measured size."""
-    out = []
-    for k, s in enumerate(sizes):
-        lo = 1 if k == 0 else int(math.sqrt(sizes[k - 1] * s)) + 1
-        hi = NMAX_INT if k == len(sizes) - 1 else int(math.sqrt(s * sizes[k + 1]))
-        out.append((lo, hi))
+def _rows(kind, precision, direction, batch, found):
+    """Table rows from the sweep's (degree, candidates, fastest one), in order
+    of the degree.  Single transforms, engines within 3 % of each other: the one
+    of the next larger degree.  Batches: pipelined from the first degree on where
+    that is faster.  Between two degrees of different engines, from 1024 on, the
+    row of the band-systolic one ends where it was measured.  Past the largest degree the
+    pipelined engine goes on: the band-systolic one's waits give up after a set
+    number of polls (about half a second), and a launch of twice the degree
+    takes eight times as long (but a triangle's hi2lo, where it is ahead at
+    every degree, keeps it)."""
+    pick = [c["cand"] for _, _, c in found]
+    for k in range(1, len(found)) if batch else range(len(found) - 2, -1, -1):
+        to = pick[k - 1 if batch else k + 1][0]
+        other = _best([r for r in found[k][1] if r["cand"][0] == to])
+        if pick[k][0] != to and other and (to == "pipeline" if batch else other["ms"] <= 1.03 * found[k][2]["ms"]):
+            pick[k] = other["cand"]
+    out, lo = [], 1
+    for k, (n, rows, _) in enumerate(found):
+        if k + 1 < len(found):
+            nx = found[k + 1][0]
+            if pick[k][0] == pick[k + 1][0] or n < 1024:
+                hi = int(math.sqrt(n * nx))
+            else:
+                hi = n if pick[k][0] == "systolic" else nx - 1
+        elif pick[k][0] == "systolic" and (kind, direction, batch) != ("tri", 0, 0):
+            hi = n
+        else:
+            hi = NMAX_INT
+        row = _row(kind, precision, direction, batch, lo, hi, pick[k])
+        if n > 2048 and row[6:] == out[-1][6:]:  # up there one row for each change
+            out[-1][5] = hi
+        else:
+            out.append(row)
+        lo = hi + 1
+    if hi < NMAX_INT:
+        pipe = _best([r for r in found[-1][1] if r["cand"][0] == "pipeline"])
+        out.append(_row(kind, precision, direction, batch, lo, NMAX_INT, pipe["cand"]))
     return out
 
 
@@ -156,36 +190,45 @@ def tune(torch, sizes=SIZES, batch_nmax=BATCH_NMAX, kinds=("sph", "tri", "disk")
         for precision in precisions:
             dt = torch.float64 if precision == 0 else torch.float32
             for direction in directions:
-                bands = _bands(sizes)
-                for n, (lo, hi) in zip(sizes, bands):
+                found = []
+                for n in sizes:
                     P = _plan(kind, n)
                     M = _full_M(kind, n)
                     X = (torch.rand(M, n, generator=g, dtype=torch.float64) - 0.5).to(dt).cuda()
-                    cands = [("systolic", p) for p in SYS_PARTS] + [("pipeline", L, W) for L, W in PIPE_SHAPES]
+                    shapes = PIPE_SHAPES if n <= 2048 else LARGE_SHAPES
+                    cands = [("systolic", p) for p in SYS_PARTS] + [("pipeline",) + s for s in shapes]
                     rows = _sweep(torch, "%s p%d d%d n=%d" % (kind, precision, direction, n), cands,
                                   lambda: [X.clone()],
                                   lambda d: ft.gpu_execute(P, direction, d[0], precision=precision))
+                    del P, X
                     best = _best(rows)
                     record["single"].append({"kind": kind, "precision": precision, "direction": direction, "n": n,
                                              "candidates": rows, "best": best})
                     if best:
-                        table.append(_row(kind, precision, direction, 0, lo, hi, best["cand"]))
-                bands = _bands(batch_nmax)
-                for nmax, (lo, hi) in zip(batch_nmax, bands):
+                        found.append((n, rows, best))
+                table += _rows(kind, precision, direction, 0, found) if found else []
+                found = []
+                for nmax in batch_nmax:
                     rng = np.random.default_rng(4242 + nmax)
-                    ns = np.round(np.exp(rng.uniform(np.log(32), np.log(nmax), batch_count))).astype(int)
+                    count = batch_count if nmax <= 1024 else batch_count // 4
+                    ns = np.round(np.exp(rng.uniform(np.log(32), np.log(nmax), count))).astype(int)
+                    if nmax > 1024:
+                        ns[0] = nmax
                     plans = [_plan(kind, int(n)) for n in ns]
                     Xs = [(torch.rand(_full_M(kind, int(n)), int(n), generator=g, dtype=torch.float64) - 0.5)
                           .to(dt).cuda() for n in ns]
-                    cands = [("pipeline",) + s for s in BATCH_SHAPES] + [("systolic", p) for p in (16, 8)]
+                    cands = [("pipeline",) + s for s in BATCH_SHAPES if s[0] > 2 or nmax <= 1024] + \
+                        [("systolic", p) for p in (16, 8)]
                     rows = _sweep(torch, "%s p%d d%d batch nmax=%d" % (kind, precision, direction, nmax), cands,
                                   lambda: [x.clone() for x in Xs],
                                   lambda d: ft.gpu_execute_batch(plans, direction, d, precision=precision))
+                    del plans, Xs
                     best = _best(rows)
                     record["batch"].append({"kind": kind, "precision": precision, "direction": direction,
-                                            "nmax": nmax, "count": batch_count, "candidates": rows, "best": best})
+                                            "nmax": nmax, "count": count, "candidates": rows, "best": best})
                     if best:
-                        table.append(_row(kind, precision, direction, 1, lo, hi, best["cand"]))
+                        found.append((nmax, rows, best))
+                table += _rows(kind, precision, direction, 1, found) if found else []
     record["table"] = table
     return record
 

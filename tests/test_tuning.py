@@ -80,6 +80,33 @@ def test_installed_tables(ft):
         ft.set_tuning_table("compiled")
 
 
+def test_compiled_table_against_the_sweep(ft):
+    """At every degree of the sweep that the package carries (single transforms
+    up to 5700, batches up to 2896) the compiled table's engine is within a
+    tenth of the fastest candidate (the margin a smaller chain part has to
+    win by), and past the sweep the band-systolic engine goes on only where it
+    was ahead at its last three degrees."""
+    import json
+    import os
+    with open(os.path.join(os.path.dirname(ft.__file__), "tuning", "gfx950.json")) as f:
+        rec = json.load(f)
+    ft.set_tuning_table("compiled")
+    last = {}
+    for batch, key, deg in ((0, "single", "n"), (1, "batch", "nmax")):
+        for x in rec[key]:
+            shape = (x["kind"], x["precision"], x["direction"], batch)
+            e, mp, L, W, wg = ft.tuned_choice(*shape, x[deg])
+            cand = ["systolic", mp] if e == ft.ENGINE_SYSTOLIC else ["pipeline", L, W] + ([wg] if batch else [])
+            ms = {tuple(c["cand"]): c["ms"] for c in x["candidates"] if c["ms"]}
+            assert ms[tuple(cand)] <= 1.1 * min(ms.values()), (shape, x[deg], cand)
+            fast = {eng: min(v for k, v in ms.items() if k[0] == eng) for eng in ("systolic", "pipeline")}
+            last.setdefault(shape, []).append((x[deg], fast["systolic"] <= fast["pipeline"]))
+    for shape, seen in last.items():
+        assert max(n for n, _ in seen) >= (2896 if shape[3] else 5700), shape
+        if ft.tuned_choice(*shape, 10000)[0] == ft.ENGINE_SYSTOLIC:
+            assert all(ahead for _, ahead in sorted(seen)[-3:]), shape
+
+
 def _rep(r):
     """A degree of the row's range, at most 700 (oracle-cheap)."""
     return max(r[4], min(r[5], 700, int(np.sqrt(r[4] * min(r[5], 4096)))))
