@@ -1668,14 +1668,16 @@ void ft_kernel_spinsph_lo2hi(const ft_spin_rotation_plan *P, const int m, ft_com
  * n, every matrix pointer and M, plus kind, direction, precision, engine and
  * tuning (L, W and the band-systolic part size).  Destroying
  * a plan that a cached schedule uses drops the schedule, and the least recently
- * used one makes room for a new list.
+ * used one makes room for a new list (of those that no graph was captured
+ * from, while there are any).
  *
  * Where only the matrices differ, a band-systolic schedule is kept and its
  * chains get the new matrices' offsets by a small kernel before the launch (48
  * spheres of degree 32 .. 512: 1.3 ms of host work to build the schedule
  * again, 5 us for the kernel), which waits for the schedule's last launch on
- * whatever stream.  A stream under capture, and any call after a launch was
- * captured (a graph may run at any time), builds a schedule as for new sizes.
+ * whatever stream.  A stream under capture, a schedule whose launch was
+ * captured (its graph may run at any time) and a pipelined one keep their
+ * matrices: the new ones get a schedule of their own, beside it.
  */
 #define FTAMD_BATCHES 8
 
@@ -1748,6 +1750,28 @@ static int batch_cache_hit(const ft_batch_cache *B, const ft_rotation_plan *cons
         if (B->dA[i] != dA[i]) *same = 0;
     }
     return 1;
+}
+
+/* The entry a call takes, and what it does with it: an entry of its list is
+ * launched as it is; else one of its plans and sizes takes its matrices, if it
+ * can (the least recently used, whose launch ended first); else an entry gets
+ * a new schedule: an empty one, or the least recently used, entries that were
+ * captured last. */
+int ftamd_batch_entry(const ftamd_batch_state *e, int n, int *action) {
+    int old = 0, rebase = -1;
+    for (int k = 0; k < n; k++) {
+        if (e[k].match == 2) {
+            *action = FTAMD_BATCH_RUN;
+            return k;
+        }
+        if (e[k].match == 1 && e[k].rebase && (rebase < 0 || e[k].used < e[rebase].used)) rebase = k;
+        if (e[k].held != e[old].held ? !e[k].held
+            : e[k].captured != e[old].captured ? !e[k].captured
+                                               : e[k].used < e[old].used)
+            old = k;
+    }
+    *action = rebase >= 0 ? FTAMD_BATCH_REBASE : FTAMD_BATCH_BUILD;
+    return rebase >= 0 ? rebase : old;
 }
 
 /* A cached band-systolic schedule on other matrices, in `stream`'s order. */
@@ -1965,38 +1989,34 @@ int ft_gpu_execute_batch(const ft_rotation_plan *const *plans, int kind, int dir
     const int L = ch.L, W = ch.W, engine = ch.engine * 2 + ch.forced, part = ch.maxpart * 16 + ch.wg_per_cu;
     pthread_mutex_lock(&g_batch_lock);
     const int capturing = ftamd_hip_capturing(stream);
-    /* a schedule of these matrices, else one of other matrices, else the least
-     * recently used entry (an empty one first) */
-    ft_batch_cache *B = NULL, *other = NULL, *old = &g_batches[0];
-    for (int k = 0; k < FTAMD_BATCHES && !B; k++) {
-        ft_batch_cache *E = &g_batches[k];
+    ftamd_batch_state st[FTAMD_BATCHES];
+    for (int k = 0; k < FTAMD_BATCHES; k++) {
+        const ft_batch_cache *E = &g_batches[k];
         int same = 0;
-        if (batch_cache_hit(E, plans, kind, direction, precision, dA, M, count, L, W, engine, part, &same)) {
-            if (same) B = E;
-            else other = E;
-        }
-        if (old->sched && (!E->sched || E->used < old->used)) old = E;
+        const int hit = batch_cache_hit(E, plans, kind, direction, precision, dA, M, count, L, W, engine, part, &same);
+        st[k].match = hit ? 1 + same : 0;
+        st[k].held = E->sched != NULL;
+        st[k].captured = E->captured;
+        st[k].rebase = hit && E->sched->sys && !E->captured && !capturing;
+        st[k].used = E->used;
     }
-    if (!B && other && other->sched->sys && !other->captured && !capturing) {
-        B = other;
+    int action = 0;
+    ft_batch_cache *B = &g_batches[ftamd_batch_entry(st, FTAMD_BATCHES, &action)];
+    if (action == FTAMD_BATCH_REBASE) {
         rc = batch_cache_rebase(B, precision, dA, count, stream);
-        if (rc != FTAMD_OK) {
-            batch_cache_clear_locked(B);
-            pthread_mutex_unlock(&g_batch_lock);
-            return rc;
-        }
-    }
-    if (!B) {
-        B = other ? other : old;
-        batch_cache_clear_locked(B);
+        if (rc != FTAMD_OK) batch_cache_clear_locked(B);
+    } else if (action == FTAMD_BATCH_BUILD) {
         ft_schedule *N = NULL;
         rc = batch_build(plans, geo, layout, direction, precision, dA, M, count, big, &ch, &N);
+        if (rc == FTAMD_OK || rc == FTAMD_ENOMEM) batch_cache_clear_locked(B);
+        if (rc == FTAMD_ENOMEM) /* with what the entry held */
+            rc = batch_build(plans, geo, layout, direction, precision, dA, M, count, big, &ch, &N);
         if (rc == FTAMD_OK)
             rc = batch_cache_store(B, N, plans, kind, direction, precision, dA, M, count, L, W, engine, part);
-        if (rc != FTAMD_OK) {
-            pthread_mutex_unlock(&g_batch_lock);
-            return rc;
-        }
+    }
+    if (rc != FTAMD_OK) {
+        pthread_mutex_unlock(&g_batch_lock);
+        return rc;
     }
     ft_schedule *S = B->sched;
     B->used = ++g_batch_calls;

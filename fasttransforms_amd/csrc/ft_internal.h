@@ -95,6 +95,17 @@ void ftamd_schedule_release(ft_schedule *S);
 void ftamd_batch_forget_plan(const ft_rotation_plan *RP);
 int ftamd_engine(void);
 
+/* A kept batch schedule, for the choice among them. */
+typedef struct {
+    int match;    /* 0: another list, 1: the call's plans, sizes and choices, 2: its matrices too */
+    int held;     /* not empty */
+    int captured; /* a launch of it was captured */
+    int rebase;   /* it can take other matrices */
+    unsigned long long used;
+} ftamd_batch_state;
+enum { FTAMD_BATCH_RUN, FTAMD_BATCH_REBASE, FTAMD_BATCH_BUILD };
+int ftamd_batch_entry(const ftamd_batch_state *e, int n, int *action);
+
 /* The engine and shape a launch uses: the knobs (ft_gpu_set_*) where set,
  * else the autotuning table's row, else the built-in choice; the pipelined
  * engine where the band-systolic one does not run the degree (unless forced). */
