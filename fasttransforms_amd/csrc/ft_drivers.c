@@ -435,6 +435,14 @@ static void pending_add(ft_schedule *S, void *stream) {
     pthread_mutex_unlock(&g_pend_lock);
 }
 
+/* Whether a launch of S on another stream waits for that stream's check. */
+static int pending_elsewhere(const ft_schedule *S, const void *stream) {
+    pthread_mutex_lock(&g_pend_lock);
+    const int r = S->pending && S->pending_stream != stream;
+    pthread_mutex_unlock(&g_pend_lock);
+    return r;
+}
+
 static void pending_remove_locked(ft_schedule *S) {
     for (int i = 0; i < g_npend; i++)
         if (g_pend[i] == S) {
@@ -1676,8 +1684,9 @@ void ft_kernel_spinsph_lo2hi(const ft_spin_rotation_plan *P, const int m, ft_com
  * spheres of degree 32 .. 512: 1.3 ms of host work to build the schedule
  * again, 5 us for the kernel), which waits for the schedule's last launch on
  * whatever stream.  A stream under capture, a schedule whose launch was
- * captured (its graph may run at any time) and a pipelined one keep their
- * matrices: the new ones get a schedule of their own, beside it.
+ * captured (its graph may run at any time), one whose launch on another
+ * stream is not checked yet (its error word is that stream's) and a pipelined
+ * one keep their matrices: the new ones get a schedule of their own, beside it.
  */
 #define FTAMD_BATCHES 8
 
@@ -1997,7 +2006,7 @@ int ft_gpu_execute_batch(const ft_rotation_plan *const *plans, int kind, int dir
         st[k].match = hit ? 1 + same : 0;
         st[k].held = E->sched != NULL;
         st[k].captured = E->captured;
-        st[k].rebase = hit && E->sched->sys && !E->captured && !capturing;
+        st[k].rebase = hit && E->sched->sys && !E->captured && !capturing && !pending_elsewhere(E->sched, stream);
         st[k].used = E->used;
     }
     int action = 0;

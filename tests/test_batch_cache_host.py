@@ -82,3 +82,34 @@ def test_captured_batch_keeps_its_schedule(ft, engine):
                 assert np.array_equal(t.cpu().numpy().T, w), k
     finally:
         ft.set_engine(ft.ENGINE_AUTO)
+
+
+@pytest.mark.gpu
+def test_a_streams_error_stays_its_own(ft):
+    """A batch whose waits expire on one stream (a limit of one poll), then the
+    same plans on other matrices on another stream: each stream's check reports
+    its own launch."""
+    import oracle as O
+    import torch
+    n = 300
+    plans = [ft.plan_rotsphere(n), ft.plan_rotsphere(n - 7)]
+    As = [O.fill("sph", P.n, 2 * P.n - 1, P.n) for P in plans]
+    A, B = ([torch.from_numpy(np.ascontiguousarray(a.T)).cuda() for a in As] for _ in range(2))
+    s1, s2 = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    ft.set_engine(ft.ENGINE_SYSTOLIC)
+    try:
+        ft.set_spin_limit(1)
+        ft.gpu_execute_batch(plans, 0, A, stream=s1)
+        torch.cuda.synchronize()
+        ft.set_spin_limit(0)
+        ft.gpu_execute_batch(plans, 0, B, stream=s2)
+        ft.synchronize(s2)
+        with pytest.raises(ft.GPUError, match="wait expired"):
+            ft.synchronize(s1)
+        ft.synchronize(s1)  # reported once
+        for P, a, b in zip(plans, As, B):
+            assert np.array_equal(b.cpu().numpy().T, O.execute(O.Plan("sph", P.n), 0, a.copy(order="F")))
+    finally:
+        ft.set_spin_limit(0)
+        ft.set_engine(ft.ENGINE_AUTO)
