@@ -11,6 +11,7 @@
  * reference's warp/permute passes (drivers.c:114-115, 125-126) have no
  * counterpart: the grouping is only a lane-to-column map.
  */
+#include <stdint.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -712,6 +713,12 @@ static int sys_upload(ft_schedule *S, const FtamdSysChain *ch, int nch, int npro
  * disk pair an order's two columns; tri and rectdisk have one per order). */
 static int sys_rowmask(int kind, int layout) { return kind != FTAMD_TRI && layout != FTAMD_LAYOUT_RECTDISK; }
 
+/* Makes the plan's band tables (its pairs uploaded; caller holds RP->lock). */
+static int sys_tables(ft_rotation_plan *RP, int dir, int precision, int S) {
+    const ft_rotation_plan *const one = RP;
+    return ftamd_sys_tables_build(&one, &one, 1, dir, precision, S, &RP->sys[dir][precision]);
+}
+
 /* Band-systolic schedule of the whole matrix (cached in the plan; caller
  * holds RP->lock).  Returns NULL with *rc == FTAMD_OK where the engine does
  * not apply. */
@@ -727,7 +734,7 @@ static ft_schedule *sys_schedule(ft_rotation_plan *RP, int layout, int dir, int 
             s->maxpart == maxpart)
             return s;
     if (!RP->sys[dir][precision]) {
-        *rc = ftamd_sys_tables_build(RP, dir, precision, Sq, &RP->sys[dir][precision]);
+        *rc = sys_tables(RP, dir, precision, Sq);
         if (*rc != FTAMD_OK) return NULL;
     }
     const ft_sys_tables *T = RP->sys[dir][precision];
@@ -1110,7 +1117,7 @@ static int tet_schedule(ft_rotation_plan *P, int part, int N, int L, int m0, int
             S = s;
             break;
         }
-    if (rc == FTAMD_OK && !S && !P->sys[dir][0]) rc = ftamd_sys_tables_build(P, dir, 0, Sq, &P->sys[dir][0]);
+    if (rc == FTAMD_OK && !S && !P->sys[dir][0]) rc = sys_tables(P, dir, 0, Sq);
     if (rc == FTAMD_OK && !S) {
         const ft_sys_tables *T = P->sys[dir][0];
         FtamdSysChain *ch = NULL;
@@ -1473,7 +1480,7 @@ static int spin_schedule(ft_spin_rotation_plan *P, int dir, int M, ft_schedule *
             S = x;
             break;
         }
-    if (rc == FTAMD_OK && !S && !R->sys[dir][0]) rc = ftamd_sys_tables_build(R, dir, 0, Sq, &R->sys[dir][0]);
+    if (rc == FTAMD_OK && !S && !R->sys[dir][0]) rc = sys_tables(R, dir, 0, Sq);
     if (rc == FTAMD_OK && !S) {
         const ft_sys_tables *T = R->sys[dir][0];
         FtamdSysChain *ch = NULL;
@@ -1861,11 +1868,71 @@ static int batch_check(const ft_rotation_plan *const *plans, int kind, int direc
     return rc;
 }
 
-/* Band-systolic schedule of a validated batch, or NULL (rc FTAMD_OK) where
- * some transform does not fit the engine or the transforms would need
- * different band widths. */
+static int cmp_plan(const void *x, const void *y) {
+    const uintptr_t a = (uintptr_t)*(void *const *)x, b = (uintptr_t)*(void *const *)y;
+    return a < b ? -1 : a > b;
+}
+
+/* The band tables of a batch's plans (tabs[i] of plans[i]), those that are
+ * missing made together: from the pairs of the largest plan, which every
+ * smaller one's are the first of (one closed form in the row and the order),
+ * or of the annulus, whose pairs come from a factorization, from each plan's
+ * own. */
+static int batch_tables(const ft_rotation_plan *const *plans, int count, const ft_rotation_plan *big, int dir,
+                        int precision, int S, ft_sys_tables **tabs) {
+    ft_rotation_plan **miss = malloc(sizeof(*miss) * 2 * (size_t)count);
+    ft_sys_tables **made = malloc(sizeof(*made) * (size_t)count);
+    int rc = miss && made ? FTAMD_OK : FTAMD_ENOMEM, n = 0, distinct = 0;
+    for (int i = 0; rc == FTAMD_OK && i < count; i++) {
+        ft_rotation_plan *RP = (ft_rotation_plan *)plans[i];
+        pthread_mutex_lock(&RP->lock);
+        if (!RP->sys[dir][precision]) miss[n++] = RP;
+        pthread_mutex_unlock(&RP->lock);
+    }
+    if (n > 0) qsort(miss, (size_t)n, sizeof(*miss), cmp_plan);
+    ft_rotation_plan **src = miss + count;
+    for (int k = 0; rc == FTAMD_OK && k < n; k++) {
+        if (k > 0 && miss[k] == miss[k - 1]) continue;
+        ft_rotation_plan *RP = miss[distinct] = miss[k];
+        src[distinct] = (ft_rotation_plan *)big;
+        if (RP->family == FTAMD_FAMILY_ANNULUS) {
+            src[distinct] = RP;
+            pthread_mutex_lock(&RP->lock);
+            rc = ftamd_plan_upload(RP, precision);
+            pthread_mutex_unlock(&RP->lock);
+        }
+        distinct++;
+    }
+    if (rc == FTAMD_OK && distinct > 0) {
+        rc = ftamd_sys_tables_build((const ft_rotation_plan *const *)miss, (const ft_rotation_plan *const *)src, distinct,
+                                    dir, precision, S, made);
+        for (int k = 0; rc == FTAMD_OK && k < distinct; k++) {
+            pthread_mutex_lock(&miss[k]->lock);
+            if (!miss[k]->sys[dir][precision]) {
+                miss[k]->sys[dir][precision] = made[k];
+                made[k] = NULL;
+            }
+            pthread_mutex_unlock(&miss[k]->lock);
+            ftamd_sys_tables_free(made[k]); /* another thread was first */
+        }
+    }
+    for (int i = 0; rc == FTAMD_OK && i < count; i++) {
+        ft_rotation_plan *RP = (ft_rotation_plan *)plans[i];
+        pthread_mutex_lock(&RP->lock);
+        tabs[i] = RP->sys[dir][precision];
+        pthread_mutex_unlock(&RP->lock);
+    }
+    free(miss);
+    free(made);
+    return rc;
+}
+
+/* Band-systolic schedule of a validated batch (big its largest plan), or NULL
+ * (rc FTAMD_OK) where some transform does not fit the engine or the transforms
+ * would need different band widths. */
 static int batch_build_sys(const ft_rotation_plan *const *plans, int kind, int layout, int direction, int precision,
-                           void *const *dA, const int *M, int count, int maxpart, ft_schedule **out) {
+                           void *const *dA, const int *M, int count, const ft_rotation_plan *big, int maxpart,
+                           ft_schedule **out) {
     *out = NULL;
     int S0 = 0;
     for (int i = 0; i < count; i++) {
@@ -1875,15 +1942,7 @@ static int batch_build_sys(const ft_rotation_plan *const *plans, int kind, int l
     }
     ft_sys_tables **tabs = malloc(sizeof(*tabs) * (size_t)count);
     if (!tabs) return FTAMD_ENOMEM;
-    int rc = FTAMD_OK;
-    for (int i = 0; rc == FTAMD_OK && i < count; i++) {
-        ft_rotation_plan *RP = (ft_rotation_plan *)plans[i];
-        pthread_mutex_lock(&RP->lock);
-        if (!RP->sys[direction][precision])
-            rc = ftamd_sys_tables_build(RP, direction, precision, S0, &RP->sys[direction][precision]);
-        tabs[i] = RP->sys[direction][precision];
-        pthread_mutex_unlock(&RP->lock);
-    }
+    int rc = batch_tables(plans, count, big, direction, precision, S0, tabs);
     FtamdSysBand *bands = NULL;
     FtamdSysChain *ch = NULL;
     int nb = 0, nch = 0, nprog = 0, *mat = NULL;
@@ -1941,7 +2000,8 @@ static int batch_build(const ft_rotation_plan *const *plans, int kind, int layou
                        void *const *dA, const int *M, int count, ft_rotation_plan *big, const ftamd_choice *ch,
                        ft_schedule **out) {
     if (ch->engine == FT_GPU_ENGINE_SYSTOLIC) {
-        int rs = batch_build_sys(plans, kind, layout, direction, precision, dA, M, count, ch->maxpart, out);
+        int rs = batch_build_sys(plans, kind, layout, direction, precision, dA, M, count, big, ch->maxpart,
+                                 out);
         if (rs != FTAMD_OK) return rs;
         if (*out) return FTAMD_OK;
         if (ch->forced) return FTAMD_EINVAL;

@@ -172,11 +172,22 @@ typedef struct {
         int jtop, jstep, K, rpar, rstep, band0, nb;
     } cls[4];
 } FtamdSysClasses;
-/* Every band's table from the plan's sines and cosines (device arrays):
- * tab[b.tab ..] of each band b, FP64 (precision 0) or rounded to FP32.  S:
- * sequences a lane; nbands <= 65535, maxsteps the most steps of a band. */
-int ftamd_hip_sys_tables(void *tab, int precision, int S, const FtamdSysClasses *c, const FtamdSysBand *bands,
-                         int nbands, int maxsteps, const double *sn, const double *cs, void *stream);
+/* A plan's tables to make: of its bands band0 .. of the launch's array, each
+ * band b's at tab[b.tab ..], the bands themselves copied to `bands` (device
+ * addresses).  The (s, c) pairs are entry 0 of the uploaded table (ft_plans.c)
+ * of a plan of degree npairs >= c.n whose pairs are this plan's. */
+typedef struct {
+    void *tab;
+    FtamdSysBand *bands;
+    const void *pairs;
+    int npairs, band0;
+    FtamdSysClasses c;
+} FtamdSysTableJob;
+/* Every band's table, FP64 (precision 0) or FP32 as the pairs are: job[b] is
+ * the job of band b (device arrays all).  S: sequences a lane; maxsteps the
+ * most steps of a band. */
+int ftamd_hip_sys_tables(const FtamdSysTableJob *jobs, const int *job, const FtamdSysBand *bands, int nbands,
+                         int maxsteps, int precision, int S, void *stream);
 /* New matrices for the chains of a batch (device arrays): chain c belongs to
  * matrix mat[c], whose offset (elements from the launch's A) becomes
  * off[mat[c]] (host array, passed by value). */

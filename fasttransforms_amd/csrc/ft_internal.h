@@ -146,7 +146,8 @@ int ftamd_spin_upload(ft_spin_rotation_plan *P);
 /* ft_systolic.c */
 int ftamd_sys_choose_S(int kind, int n, int precision);
 int ftamd_sys_applies(int kind, int n, int dir, int precision);
-int ftamd_sys_tables_build(const ft_rotation_plan *RP, int dir, int precision, int S, ft_sys_tables **out);
+int ftamd_sys_tables_build(const ft_rotation_plan *const *plans, const ft_rotation_plan *const *src, int count,
+                           int dir, int precision, int S, ft_sys_tables **out);
 void ftamd_sys_tables_free(ft_sys_tables *T);
 int ftamd_sys_tables_S(const ft_sys_tables *T);
 const void *ftamd_sys_tables_dev_bands(const ft_sys_tables *T);

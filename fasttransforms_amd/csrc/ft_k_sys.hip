@@ -29,18 +29,24 @@ extern "C" int ftamd_hip_sys_launch(const FtamdSysLaunch *a, int precision, int 
 namespace ftsys {
 
 // A thread writes the entry of one step and sequence of a band (blockIdx.y).
-// Bound by the bus that brings the sines and cosines (n = 2048, FP64: 33 MB,
-// and 39 MB of tables; on the host, entry by entry, 45 ms).
+// The values come from the pairs that the plans' upload left on the device, and
+// the plans of a batch are one launch: with an upload of the sines and cosines,
+// two allocations and a wait for each plan, 48 spheres of degree 32 .. 1024
+// took 11.3 ms on their first call, half of it here.  Bound by the 39 MB of
+// tables at n = 2048 in FP64 (on the host, entry by entry, 45 ms).
 template <typename T>
-__global__ void __launch_bounds__(256) tables_kernel(Pair<T> *tab, int S, FtamdSysClasses c, const FtamdSysBand *bands,
-                                                     const double *sn, const double *cs) {
-    const int b = blockIdx.y, B = kLanes * S;
+__global__ void __launch_bounds__(256) tables_kernel(const FtamdSysTableJob *jobs, const int *job,
+                                                     const FtamdSysBand *bands, int b0, int S) {
+    const int b = b0 + blockIdx.y, B = kLanes * S;
     const FtamdSysBand bd = bands[b];
+    const FtamdSysTableJob &jb = jobs[job[b]];
     const long long x = blockIdx.x * 256LL + threadIdx.x;
     const int t = (int)(x / B), q = (int)(x % B);
     if (t >= bd.steps + FTAMD_SYS_PREFETCH) return;
+    if (x == 0) jb.bands[b - jb.band0] = bd;
+    const FtamdSysClasses &c = jb.c;
     int k = 0;
-    while (k + 1 < c.ncls && b >= c.cls[k + 1].band0) ++k;
+    while (k + 1 < c.ncls && b - jb.band0 >= c.cls[k + 1].band0) ++k;
     const auto cl = c.cls[k];
     Pair<T> v{T(0), T(1)};
     if (q < bd.nseq) {
@@ -53,14 +59,19 @@ __global__ void __launch_bounds__(256) tables_kernel(Pair<T> *tab, int S, FtamdS
                         : c.kind == FTAMD_TRI ? c.n - 2 - j
                                               : c.n - 2 - (j + 1) / 2;
         if (e >= 0 && e <= top) {
-            const long long row = cl.rstep * e + cl.rpar, n = c.n;
-            const long long ix = c.kind == FTAMD_DISK ? row + j * n - (long long)(j / 2) * ((j + 1) / 2)
-                                                      : row + j * (2 * n + 1 - j) / 2;
-            v = Pair<T>{(T)sn[ix], (T)cs[ix]};
+            // the pair's place (ftamd_plan_upload: a sphere's column holds its even rows first)
+            const long long n = jb.npairs;
+            const int row = cl.rstep * e + cl.rpar;
+            const int at = c.kind == FTAMD_SPH && (row & 1) ? (jb.npairs - j + 1) / 2 + row / 2
+                           : c.kind == FTAMD_SPH            ? row / 2
+                                                            : row;
+            const long long col = c.kind == FTAMD_DISK ? j * n - (long long)(j / 2) * ((j + 1) / 2)
+                                                       : j * (2 * n + 1 - j) / 2;
+            v = ((const Pair<T> *)jb.pairs)[col + at];
         }
     }
     const int lane = q / S, s = q % S;
-    tab[bd.tab + (long long)t * B + (FTAMD_SYS_SLOT_MAJOR(sizeof(T) == 4) ? s * kLanes + lane : q)] = v;
+    ((Pair<T> *)jb.tab)[bd.tab + (long long)t * B + (FTAMD_SYS_SLOT_MAJOR(sizeof(T) == 4) ? s * kLanes + lane : q)] = v;
 }
 
 // The offsets of a batch's matrices (elements from the launch's A), passed by value.
@@ -79,19 +90,17 @@ __global__ void __launch_bounds__(256) rebase_kernel(FtamdSysChain *chains, cons
 
 }  // namespace ftsys
 
-extern "C" int ftamd_hip_sys_tables(void *tab, int precision, int S, const FtamdSysClasses *c,
-                                    const FtamdSysBand *bands, int nbands, int maxsteps, const double *sn,
-                                    const double *cs, void *stream) {
-    if (nbands <= 0) return FTAMD_OK;
-    if (nbands > 65535 || S < 1 || maxsteps < 0 || c->ncls < 1 || c->ncls > 4) return FTAMD_EINVAL;
+extern "C" int ftamd_hip_sys_tables(const FtamdSysTableJob *jobs, const int *job, const FtamdSysBand *bands,
+                                    int nbands, int maxsteps, int precision, int S, void *stream) {
+    if (S < 1 || maxsteps < 0 || nbands < 0) return FTAMD_EINVAL;
     const long long entries = (long long)(maxsteps + FTAMD_SYS_PREFETCH) * ftsys::kLanes * S;
-    const dim3 grid((unsigned)((entries + 255) / 256), nbands), block(256);
-    if (precision == 0)
-        hipLaunchKernelGGL(ftsys::tables_kernel<double>, grid, block, 0, (hipStream_t)stream,
-                           (ftsys::Pair<double> *)tab, S, *c, bands, sn, cs);
-    else
-        hipLaunchKernelGGL(ftsys::tables_kernel<float>, grid, block, 0, (hipStream_t)stream, (ftsys::Pair<float> *)tab,
-                           S, *c, bands, sn, cs);
+    for (int b0 = 0; b0 < nbands; b0 += 65535) {
+        const dim3 grid((unsigned)((entries + 255) / 256), nbands - b0 < 65535 ? nbands - b0 : 65535), block(256);
+        if (precision == 0)
+            hipLaunchKernelGGL(ftsys::tables_kernel<double>, grid, block, 0, (hipStream_t)stream, jobs, job, bands, b0, S);
+        else
+            hipLaunchKernelGGL(ftsys::tables_kernel<float>, grid, block, 0, (hipStream_t)stream, jobs, job, bands, b0, S);
+    }
     hipError_t e = hipGetLastError();
     return e == hipSuccess ? FTAMD_OK : FTAMD_EDEVICE;
 }

@@ -80,8 +80,8 @@ struct ft_sys_tables {
     int band0[4], nb[4];     /* bands of class c: band0[c] .. band0[c]+nb[c]-1 */
     FtamdSysBand *bands;     /* host copy */
     int nbands;
+    void *d_tab;             /* the tables, then the bands (one allocation) */
     void *d_bands;
-    void *d_tab;
 };
 
 int ftamd_sys_tables_S(const ft_sys_tables *T) { return T->S; }
@@ -91,7 +91,6 @@ const FtamdSysBand *ftamd_sys_tables_host_bands(const ft_sys_tables *T) { return
 
 void ftamd_sys_tables_free(ft_sys_tables *T) {
     if (!T) return;
-    ftamd_hip_free(T->d_bands);
     ftamd_hip_free(T->d_tab);
     free(T->bands);
     free(T);
@@ -222,54 +221,77 @@ static int tables_host(const ft_rotation_plan *RP, int dir, int S, ft_sys_tables
     return FTAMD_OK;
 }
 
-int ftamd_sys_tables_build(const ft_rotation_plan *RP, int dir, int precision, int S, ft_sys_tables **out) {
-    *out = NULL;
-    ft_sys_tables *T = calloc(1, sizeof(ft_sys_tables));
-    if (!T) return FTAMD_ENOMEM;
-    long long entries = 0;
-    int rc = tables_bands(RP, dir, precision, S, T, &entries);
-    size_t esz = precision == 0 ? sizeof(double) : sizeof(float);
-    if (rc == FTAMD_OK && !ftamd_sys_applies(RP->kind, RP->n, dir, precision)) rc = FTAMD_EINVAL;
-    if (rc == FTAMD_OK) rc = ftamd_hip_malloc(&T->d_tab, (size_t)(entries > 0 ? entries : 1) * 2 * esz);
-    if (rc == FTAMD_OK)
-        rc = ftamd_hip_malloc(&T->d_bands, sizeof(FtamdSysBand) * (size_t)(T->nbands > 0 ? T->nbands : 1));
-    if (rc == FTAMD_OK && T->nbands > 0) {
-        const size_t bytes = sizeof(double) * (size_t)RP->nsc;
-        FtamdSysClasses c;
-        memset(&c, 0, sizeof(c));
-        c.kind = RP->kind;
-        c.n = RP->n;
-        c.dir = dir;
-        c.ncls = T->ncls;
-        int maxsteps = 0;
-        for (int k = 0; k < T->ncls; k++) {
-            c.cls[k].jtop = T->cls[k].jtop;
-            c.cls[k].jstep = T->cls[k].jstep;
-            c.cls[k].K = T->cls[k].K;
-            c.cls[k].rpar = T->cls[k].rpar;
-            c.cls[k].rstep = T->cls[k].rstep;
-            c.cls[k].band0 = T->band0[k];
-            c.cls[k].nb = T->nb[k];
-        }
+/* The tables of `count` distinct plans for one direction, precision and S, in
+ * one upload and one launch: plan i's from the uploaded pairs of src[i], a plan
+ * of at least its degree with the same pairs.  out[i] gets each; on an error
+ * all are NULL. */
+int ftamd_sys_tables_build(const ft_rotation_plan *const *plans, const ft_rotation_plan *const *src, int count,
+                           int dir, int precision, int S, ft_sys_tables **out) {
+    const size_t pair = 2 * (precision == 0 ? sizeof(double) : sizeof(float));
+    int rc = FTAMD_OK, nbands = 0, maxsteps = 0;
+    for (int i = 0; i < count; i++) out[i] = NULL;
+    for (int i = 0; rc == FTAMD_OK && i < count; i++) {
+        long long entries = 0;
+        if (!ftamd_sys_applies(plans[i]->kind, plans[i]->n, dir, precision)) rc = FTAMD_EINVAL;
+        ft_sys_tables *T = out[i] = rc == FTAMD_OK ? calloc(1, sizeof(ft_sys_tables)) : NULL;
+        if (rc == FTAMD_OK) rc = T ? tables_bands(plans[i], dir, precision, S, T, &entries) : FTAMD_ENOMEM;
+        if (rc != FTAMD_OK) break;
+        const size_t tab = ((size_t)entries * pair + 255) & ~(size_t)255;
+        rc = ftamd_hip_malloc(&T->d_tab, tab + sizeof(FtamdSysBand) * (size_t)T->nbands + 1);
+        if (rc == FTAMD_OK) T->d_bands = (char *)T->d_tab + tab;
+        nbands += T->nbands;
         for (int b = 0; b < T->nbands; b++)
             if (T->bands[b].steps > maxsteps) maxsteps = T->bands[b].steps;
-        char *sc = NULL; /* the plan's sines, then its cosines */
-        rc = ftamd_hip_h2d(T->d_bands, T->bands, sizeof(FtamdSysBand) * (size_t)T->nbands, NULL);
-        if (rc == FTAMD_OK) rc = ftamd_hip_malloc((void **)&sc, 2 * bytes);
-        if (rc == FTAMD_OK) rc = ftamd_hip_h2d(sc, RP->s, bytes, NULL);
-        if (rc == FTAMD_OK) rc = ftamd_hip_h2d(sc + bytes, RP->c, bytes, NULL);
+    }
+    /* the bands of all plans, the jobs, each band's job */
+    const size_t obj = sizeof(FtamdSysBand) * (size_t)nbands, oj = obj + sizeof(FtamdSysTableJob) * (size_t)count;
+    const size_t bytes = oj + sizeof(int) * (size_t)nbands;
+    char *h = rc == FTAMD_OK && nbands > 0 ? calloc(1, bytes) : NULL, *d = NULL;
+    if (rc == FTAMD_OK && nbands > 0) rc = h ? ftamd_hip_malloc((void **)&d, bytes) : FTAMD_ENOMEM;
+    if (rc == FTAMD_OK && nbands > 0) {
+        FtamdSysBand *bands = (FtamdSysBand *)h;
+        FtamdSysTableJob *jobs = (FtamdSysTableJob *)(h + obj);
+        int *job = (int *)(h + oj);
+        for (int i = 0, b = 0; i < count; i++) {
+            const ft_sys_tables *T = out[i];
+            FtamdSysTableJob *J = &jobs[i];
+            J->tab = T->d_tab;
+            J->bands = T->d_bands;
+            J->pairs = ftamd_plan_table(src[i], precision);
+            J->npairs = src[i]->n;
+            J->band0 = b;
+            J->c.kind = plans[i]->kind;
+            J->c.n = plans[i]->n;
+            J->c.dir = dir;
+            J->c.ncls = T->ncls;
+            for (int k = 0; k < T->ncls; k++) {
+                J->c.cls[k].jtop = T->cls[k].jtop;
+                J->c.cls[k].jstep = T->cls[k].jstep;
+                J->c.cls[k].K = T->cls[k].K;
+                J->c.cls[k].rpar = T->cls[k].rpar;
+                J->c.cls[k].rstep = T->cls[k].rstep;
+                J->c.cls[k].band0 = T->band0[k];
+                J->c.cls[k].nb = T->nb[k];
+            }
+            for (int k = 0; k < T->nbands; k++, b++) {
+                bands[b] = T->bands[k];
+                job[b] = i;
+            }
+        }
+        rc = ftamd_hip_h2d(d, h, bytes, NULL);
         if (rc == FTAMD_OK)
-            rc = ftamd_hip_sys_tables(T->d_tab, precision, S, &c, (const FtamdSysBand *)T->d_bands, T->nbands, maxsteps,
-                                      (const double *)sc, (const double *)(sc + bytes), NULL);
-        if (rc == FTAMD_OK) rc = ftamd_hip_sync(NULL);
-        ftamd_hip_free(sc);
+            rc = ftamd_hip_sys_tables((const FtamdSysTableJob *)(d + obj), (const int *)(d + oj), (const FtamdSysBand *)d,
+                                      nbands, maxsteps, precision, S, NULL);
+        const int rs = ftamd_hip_sync(NULL);
+        if (rc == FTAMD_OK) rc = rs;
     }
-    if (rc != FTAMD_OK) {
-        ftamd_sys_tables_free(T);
-        return rc;
+    ftamd_hip_free(d);
+    free(h);
+    for (int i = 0; rc != FTAMD_OK && i < count; i++) {
+        ftamd_sys_tables_free(out[i]);
+        out[i] = NULL;
     }
-    *out = T;
-    return FTAMD_OK;
+    return rc;
 }
 
 static int cmp_nb_desc(const void *x, const void *y) {
