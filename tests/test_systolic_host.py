@@ -114,3 +114,21 @@ def test_degrees_past_the_tables(ft, kind, precision, direction, n):
         ft.set_engine(ft.ENGINE_AUTO)
         ft.set_tuning_table("compiled")
     assert ft.tuned_choice(kind, precision, direction, 0, 2 * n)[0] == ft.ENGINE_PIPELINE
+
+
+@pytest.mark.parametrize("kind,n,nsx", [("sph", 90, 1), ("sph", 200, 7), ("sph", 200, 64), ("tri", 150, 5), ("disk", 120, 8),
+                                        ("disk", 120, 33)])
+@pytest.mark.parametrize("d", [0, 1])
+def test_whole_chains_go_to_the_least_loaded_slot(ft, kind, n, nsx, d):
+    """Whole chains on one list of slots: each in turn goes to the first of the
+    slots with the fewest steps so far."""
+    P, _ = _plan(ft, kind, n, CASES[[k for k, _ in CASES].index(kind)][1])
+    M = {"sph": 2 * n - 1, "tri": n, "disk": 4 * n - 3}[kind]
+    bands, _, chains = se.host_build(ft._lib, P.ptr, d, 2, M, 16)
+    assert all(c.split_in < 0 and c.split_out < 0 for c in chains) and len(chains) > nsx
+    items, slot_items, _ = se.assign(ft._lib, bands, chains, 1, nsx)
+    slot = {items[k][0]: s for s in range(nsx) for k in range(slot_items[s], slot_items[s + 1])}
+    load = [0] * nsx
+    for c, ch in enumerate(chains):
+        assert slot[c] == load.index(min(load)), c
+        load[slot[c]] += sum(b.steps for b in bands[ch.band0:ch.band0 + ch.nb])
