@@ -79,12 +79,20 @@ bool ftamd_dft_fits(int len) {
     return len >= 1 && (len <= FTAMD_DFT_MAX || len == 2 * FTAMD_DFT_MAX);
 }
 
+static bool by_chirp(int len) { return len < 64 || (len & (len - 1)) != 0; }
+
+int ftamd_dft_points(int len) {
+    int points = 64;
+    while (points < (by_chirp(len) ? 2 * len - 1 : len)) points *= 2;
+    return points;
+}
+
 int ftamd_dft_create(int len, FtamdDft **out) {
     *out = NULL;
     if (!ftamd_dft_fits(len)) return FTAMD_EINVAL;
-    const bool chirp = len < 64 || (len & (len - 1)) != 0;
+    const bool chirp = by_chirp(len);
     int logl = 6;
-    while ((1 << logl) < (chirp ? 2 * len - 1 : len)) ++logl;
+    while ((1 << logl) < ftamd_dft_points(len)) ++logl;
     FtamdDft *d = (FtamdDft *)calloc(1, sizeof(FtamdDft));
     if (!d) return FTAMD_ENOMEM;
     d->len = len;

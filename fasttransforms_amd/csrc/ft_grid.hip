@@ -14,8 +14,8 @@
 //
 // The sphere's, the vector field's, the annulus's and the disk's grids take
 // two launches of the line transforms (ft_dft.hpp).  Lengths those do not
-// take (above FTAMD_DFT_MAX), the disk's DCT-IV and the other geometries run
-// hipFFT between kernels: there the synthesis plans put two columns in one
+// take (above FTAMD_DFT_MAX) or take longer for (ftamd_grid_lines), the disk's
+// DCT-IV and the other geometries run hipFFT between kernels: there the synthesis plans put two columns in one
 // FFT, and the phi DFTs are hipFFT's strided transforms (row i is the
 // transform at element i, stride N); with N even, rows 2p and 2p+1 share one
 // complex DFT over X read as N/2 x M complex.
@@ -451,6 +451,33 @@ static int phi_plan_pair(FtamdGrid *g) {
     return fft_ok(hipfftPlanMany(&g->phi, 1, n2, n2, P, 1, n2, P, 1, HIPFFT_Z2Z, P));
 }
 
+// Whether the line transforms run an N x M grid (sphere, vector field,
+// annulus, disk): where they take both lengths, but for pairs of lengths of
+// primes up to 7 alone, which hipFFT transforms without a convolution.  There
+// it depends on what the convolutions waste: their points over the length, a
+// convolution of 8192 points (one workgroup a CU, and with few rows the time
+// of one line) counted more, against a bound for each kind of grid (odd N:
+// hipFFT takes rows one by one; the disk's has passes more).  Synthesis, us by
+// lines / hipFFT: N = 1120, M = 1125 57 / 45, 600 x 1215 35 / 32, 1200 x 2401
+// 131 / 85, 2250 x 1215 132 / 82, 64 x 2187 32 / 24; 1000 x 1575 44 / 53, 1875
+// x 1875 85 / 143, 1920 x 3645 194 / 194; disk 1200 x 2401 171 / 141, 1080 x
+// 1875 98 / 98, 1000 x 1323 66 / 79.  With another prime in either length lines
+// win: 2500 x 1009 93 / 93, 1009 x 2187 91 / 131, 1094 x 2187 127 / 148.  Below
+// 1024 points both take what their launches take.
+extern "C" int ftamd_grid_lines(int N, int M, int disk) {
+    if (!ftamd_dft_fits(N) || !ftamd_dft_fits(M)) return 0;
+    auto smooth = [](int len) {
+        for (int p = 2; p <= 7; ++p)
+            while (len % p == 0) len /= p;
+        return len == 1;
+    };
+    const int pn = ftamd_dft_points(N), pm = ftamd_dft_points(M);
+    if (!smooth(N) || !smooth(M) || (pn < 1024 && pm < 1024)) return 1;
+    const double wn = (double)pn / N * (pn > N && pn > 4096 ? 2.4 : 1.0);
+    const double wm = (double)pm / M * (pm > M && pm > 4096 ? (N > 128 ? 1.6 : 3.0) : 1.0);
+    return wn + wm < (N % 2 ? 8.0 : disk ? 6.5 : 5.9);
+}
+
 extern "C" int ftamd_grid_create(int N, int M, int type3, int plan_mode, const double *w, FtamdGrid **out) {
     *out = NULL;
     /* columns are the launch grid's y dimension (at most 65535) */
@@ -478,7 +505,7 @@ extern "C" int ftamd_grid_create(int N, int M, int type3, int plan_mode, const d
         tw[k] = make_double2((double)cosl(th), (double)sinl(th));
     }
     if (rc == FTAMD_OK && hipMalloc((void **)&g->tw, sizeof(double2) * (size_t)N) != hipSuccess) rc = FTAMD_ENOMEM;
-    const bool lines = ftamd_dft_fits(N) && ftamd_dft_fits(M);
+    const bool lines = ftamd_grid_lines(N, M, plan_mode == 2);
     if (lines) {
         if (rc == FTAMD_OK) rc = ftamd_dft_create(N, &g->dft_theta);
         if (rc == FTAMD_OK) rc = ftamd_dft_create(M, &g->dft_phi);

@@ -13,6 +13,7 @@
 constexpr int FTAMD_DFT_MAX = 4096;
 struct FtamdDft;
 bool ftamd_dft_fits(int len);
+int ftamd_dft_points(int len);  // of its power-of-two DFTs: len, or the convolution's
 int ftamd_dft_create(int len, FtamdDft **out);
 void ftamd_dft_destroy(FtamdDft *d);
 
