@@ -253,6 +253,22 @@ static double column_rotations(int kind, int n, int jmin, int jmax) {
 
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
+typedef struct {
+    double key;
+    int g;
+} ft_rank;
+
+static int cmp_rank(const void *x, const void *y) {
+    const ft_rank *a = x, *b = y;
+    return a->key > b->key ? -1 : a->key < b->key ? 1 : a->g - b->g;
+}
+
+/* The groups by decreasing key, equal ones in their order. */
+static void rank_order(ft_rank *rank, int G, int *order) {
+    qsort(rank, (size_t)G, sizeof(ft_rank), cmp_rank);
+    for (int a = 0; a < G; a++) order[a] = rank[a].g;
+}
+
 /*
  * Upload groups, lane maps, the task order and a zeroed workspace.
  *
@@ -269,17 +285,15 @@ static int finish_schedule(ft_schedule *S, ft_hgroup *gs, int G, int nprog, cons
     for (int g = 0; g < G; g++)
         if (gs[g].g.npass > maxpass) maxpass = gs[g].g.npass;
     int *order = malloc(sizeof(int) * (size_t)(G ? G : 1));
-    if (!order) return FTAMD_ENOMEM;
-    /* LPT assignment of groups to XCDs */
-    for (int g = 0; g < G; g++) order[g] = g;
-    for (int a = 1; a < G; a++) {
-        int v = order[a], b = a - 1;
-        while (b >= 0 && gs[order[b]].work < gs[v].work) {
-            order[b + 1] = order[b];
-            b--;
-        }
-        order[b + 1] = v;
+    ft_rank *rank = malloc(sizeof(ft_rank) * (size_t)(G ? G : 1));
+    if (!order || !rank) {
+        free(order);
+        free(rank);
+        return FTAMD_ENOMEM;
     }
+    /* LPT assignment of groups to XCDs */
+    for (int g = 0; g < G; g++) rank[g] = (ft_rank){gs[g].work, g};
+    rank_order(rank, G, order);
     double load[FTAMD_MAX_XCD] = {0};
     for (int a = 0; a < G; a++) {
         int best = 0;
@@ -289,15 +303,9 @@ static int finish_schedule(ft_schedule *S, ft_hgroup *gs, int G, int nprog, cons
         load[best] += gs[order[a]].work;
     }
     /* within an XCD: pass-major, longest chains first */
-    for (int g = 0; g < G; g++) order[g] = g;
-    for (int a = 1; a < G; a++) {
-        int v = order[a], b = a - 1;
-        while (b >= 0 && gs[order[b]].crit < gs[v].crit) {
-            order[b + 1] = order[b];
-            b--;
-        }
-        order[b + 1] = v;
-    }
+    for (int g = 0; g < G; g++) rank[g] = (ft_rank){gs[g].crit, g};
+    rank_order(rank, G, order);
+    free(rank);
     /* issue priority by chain length, and the boundary buffers: npass-1 of
      * [rows of the sub-problem][64 lanes] per group */
     int maxcrit = 1;
