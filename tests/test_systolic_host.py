@@ -132,3 +132,40 @@ def test_whole_chains_go_to_the_least_loaded_slot(ft, kind, n, nsx, d):
     for c, ch in enumerate(chains):
         assert slot[c] == load.index(min(load)), c
         load[slot[c]] += sum(b.steps for b in bands[ch.band0:ch.band0 + ch.nb])
+
+
+@pytest.mark.parametrize("kind,params", CASES[:2] + CASES[3:])
+@pytest.mark.parametrize("d", [0, 1])
+def test_table_steps_a_band_requests(ft, kind, params, d):
+    """The kernel's requests for table steps (ft_systolic.hpp, run_band) stay
+    inside the tables, FP64 (8 steps staged ahead) and FP32 (16, the source
+    clamped to the table's last block): band w of a part starts idle(w) steps
+    before its table, in the spare steps of the band before it, and runs blocks
+    of 8 until its last position is stored; what lies outside a band's own
+    rotations are identities."""
+    U, PF, LAG = 8, 16, 3 * 15 + 2 + 1
+    rng = np.random.default_rng(5)
+    for n in list(range(3, 76)) + [int(v) for v in rng.integers(76, 400, 12)]:
+        P, _ = _plan(ft, kind, n, params)
+        M = {"sph": 2 * n - 1, "tri": n, "disk": 4 * n - 3}[kind]
+        for maxpart in (1, 3, 16):
+            bands, tab, chains = se.host_build(ft._lib, P.ptr, d, 2, M, maxpart)
+            ends = {b.tab + (b.steps + PF) * 32 for b in bands}
+            for ch in chains:
+                for w in range(ch.nb):
+                    b, off = bands[ch.band0 + w], (2 * w) % U
+                    if off:
+                        assert b.tab in ends, "a band before it"
+                        before = tab[b.tab - off * 32:b.tab]
+                        assert (before == (0.0, 1.0)).all()
+                    total = (b.R + off + LAG + U) // U * U
+                    for staged in (8, 16):
+                        last = b.steps + PF - U + off
+                        src = [t + staged for t in range(0, total, U)]
+                        if staged == 16:
+                            src = [min(s, last) for s in src]
+                        assert max(src) - off + U <= b.steps + PF, (n, w, staged)
+                        assert staged - off <= b.steps + PF
+                    # a step past the last rotation of the band's last sequence
+                    tail = tab[b.tab + (b.R + LAG) * 32:b.tab + (b.steps + PF) * 32]
+                    assert (tail == (0.0, 1.0)).all(), (n, w)
