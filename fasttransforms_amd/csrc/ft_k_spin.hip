@@ -181,9 +181,9 @@ __device__ void sweep(const Args &a, const Column &lq, const Column &cq, int jl,
         if (lvalid && t >= 0 && t <= RL)
             lA[(long long)(DIR == 0 ? RL - t : t) * a.row_stride] = sh.rows[S][lcol * PITCH + lk];
     };
-    for (int g = 0; g < rounds; g += 2) {  // a round past the end stores nothing
+    for (int g = 0; g < rounds; g += 2) {
         round(g, v0);
-        round(g + 1, v1);
+        if (g + 1 < rounds) round(g + 1, v1);
     }
     __threadfence_block();  // the next sweep's loads take rows that other lanes stored
     __syncthreads();
