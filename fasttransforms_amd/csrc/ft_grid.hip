@@ -453,26 +453,50 @@ static int phi_plan_pair(FtamdGrid *g) {
 
 // Whether the line transforms run an N x M grid (sphere, vector field,
 // annulus, disk): where they take both lengths, but for pairs of lengths of
-// primes up to 7 alone, which hipFFT transforms without a convolution.  There
-// it depends on what the convolutions waste: their points over the length, a
-// convolution of 8192 points (one workgroup a CU, and with few rows the time
-// of one line) counted more, against a bound for each kind of grid (odd N:
-// hipFFT takes rows one by one; the disk's has passes more).  Synthesis, us by
-// lines / hipFFT: N = 1120, M = 1125 57 / 45, 600 x 1215 35 / 32, 1200 x 2401
-// 131 / 85, 2250 x 1215 132 / 82, 64 x 2187 32 / 24; 1000 x 1575 44 / 53, 1875
-// x 1875 85 / 143, 1920 x 3645 194 / 194; disk 1200 x 2401 171 / 141, 1080 x
-// 1875 98 / 98, 1000 x 1323 66 / 79.  With another prime in either length lines
-// win: 2500 x 1009 93 / 93, 1009 x 2187 91 / 131, 1094 x 2187 127 / 148.  Below
-// 1024 points both take what their launches take.
+// primes up to 17 alone, which hipFFT transforms without a convolution.  Of
+// those they run the ones they are no further off on and no slower.
+//
+// The error: each side's square goes with its passes, hipFFT's with the primes
+// (by the radix, fitted to 150 pairs against long double, in 1e-32 of the
+// relative 2-norm), the convolutions' with the logarithm of their points (less
+// where N is a power of two and has none).  With lengths up to 256 the fit does
+// not tell them apart: there hipFFT is taken unless N is such a power.  Relative
+// errors of the synthesis by lines / hipFFT, 1e-16: 39 x 51 3.3 / 2.8 (analysis
+// 4.3 / 3.0), 85 x 121 3.5 / 2.7, 715 x 825 4.4 / 3.9; 128 x 231 3.3 / 4.0, 360 x
+// 539 3.9 / 5.0, 1000 x 1215 (analysis) 4.6 / 5.2.  With another prime in
+// either length hipFFT has convolutions too and lines are closer: 67 x 133
+// (analysis) 3.7 / 7.8, 600 x 1199 4.9 / 7.5.
+//
+// The time, with primes up to 7: it depends on what the convolutions waste,
+// their points over the length, a convolution of 8192 points (one workgroup a
+// CU, and with few rows the time of one line) counted more, against a bound for
+// each kind of grid (odd N: hipFFT takes rows one by one; the disk's has passes
+// more).  Synthesis, us by lines / hipFFT: N = 1120, M = 1125 57 / 45, 600 x
+// 1215 35 / 32, 1200 x 2401 131 / 85, 2250 x 1215 132 / 82, 64 x 2187 32 / 24;
+// 1000 x 1575 44 / 53, 512 x 945 23 / 28, 1875 x 2401 173 / 201; disk 1200 x
+// 2401 171 / 141, 1000 x 1323 66 / 79.  With another prime in either length
+// lines win: 2500 x 1009 93 / 93, 1009 x 2187 91 / 131, 1094 x 2187 127 / 148.
 extern "C" int ftamd_grid_lines(int N, int M, int disk) {
     if (!ftamd_dft_fits(N) || !ftamd_dft_fits(M)) return 0;
-    auto smooth = [](int len) {
-        for (int p = 2; p <= 7; ++p)
-            while (len % p == 0) len /= p;
-        return len == 1;
+    const int prime[] = {2, 3, 5, 7, 11, 13, 17};
+    const double err[] = {1.45, 1.85, 2.06, 4.2, 2.3, 3.2, 3.7};
+    double hip = 0;
+    int most = 0;
+    auto rest = [&](int len) {
+        for (int k = 0; k < 7; ++k)
+            for (; len % prime[k] == 0; len /= prime[k]) {
+                hip += err[k];
+                most = prime[k] > most ? prime[k] : most;
+            }
+        return len;
     };
+    const int other = rest(N) * rest(M);
+    if (other > 1) return 1;
     const int pn = ftamd_dft_points(N), pm = ftamd_dft_points(M);
-    if (!smooth(N) || !smooth(M) || (pn < 1024 && pm < 1024)) return 1;
+    if (N <= 256 && M <= 256) return N >= 128 && pn == N;
+    const double lines = 0.9 * log2((double)pn) + 0.68 * log2((double)pm) - (pn == N ? 1.9 : 0.15);
+    if (lines > 0.83 * hip) return 0;
+    if (most > 7) return 1;
     const double wn = (double)pn / N * (pn > N && pn > 4096 ? 2.4 : 1.0);
     const double wm = (double)pm / M * (pm > M && pm > 4096 ? (N > 128 ? 1.6 : 3.0) : 1.0);
     return wn + wm < (N % 2 ? 8.0 : disk ? 6.5 : 5.9);

@@ -292,7 +292,7 @@ int ft_gpu_execute_tet(const ft_rotation_plan *RP1, const ft_rotation_plan *RP2,
  * N x M grid theta_i = (i+1/2) pi / N, phi_j = 2 pi j / M) and analysis (the
  * inverse) on the sphere, and their vector-field variants, on the GPU
  * (this library's kernels in place of FFTW; hipFFT for lines longer than 4096
- * and for some N and M of primes up to 7).  The plan holds device work buffers
+ * and for some N and M of primes up to 17).  The plan holds device work buffers
  * (about 8 N M bytes, 24 N M with hipFFT); flags are ignored.  X is N x M
  * column-major, host or device, M odd, overwritten in place.  Synthesis 'N'
  * and analysis 'T' take a synthesis plan, synthesis 'T' and analysis 'N' an

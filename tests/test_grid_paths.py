@@ -20,9 +20,7 @@ SIZES = [
     (1000, 1575, 0, 1),  # 44.0 / 52.7
     (1344, 2025, 0, 1),  # 67.5 / 78.9
     (512, 945, 0, 1),    # 23.1 / 27.7
-    (64, 125, 0, 1),     # 12.1 / 15.1
-    (126, 225, 0, 1),    # 14.6 / 15.0
-    (675, 1215, 0, 1),   # 38.5 / 51.6
+    (1875, 1875, 0, 0),  # 85.1 / 143, by the error
     (1875, 2401, 0, 1),  # 173 / 201
     (2048, 3125, 0, 1),  # 162 / 173
     (1024, 2047, 0, 1),  # 46.3 / 96.7
@@ -32,10 +30,36 @@ SIZES = [
     (8192, 255, 0, 1),   # 49.4 / 58.9
     (1200, 2401, 1, 0),  # 171 / 141
     (2250, 63, 1, 0),    # 53.6 / 42.1
-    (1080, 1875, 1, 1),  # 98.2 / 97.7
     (1000, 1323, 1, 1),  # 65.6 / 78.8
     (4097, 63, 0, 0), (63, 4097, 0, 0),  # longer than the lines
 ]
+
+
+# N, M, lines: relative errors of the analysis, 1e-16, by the lines and by hipFFT
+ERRORS = [
+    (25, 33, 0),    # 3.5 / 2.7
+    (39, 51, 0),    # 4.3 / 3.0
+    (64, 125, 0),   # 3.8 / 3.75
+    (100, 105, 0),  # 4.7 / 3.9
+    (85, 121, 0),   # 4.2 / 3.2
+    (125, 231, 0),  # 4.0 / 4.3, synthesis 3.9 / 3.3
+    (400, 625, 0),  # 4.6 / 4.3
+    (500, 845, 0),  # 4.8 / 4.3
+    (715, 825, 0),  # 4.8 / 4.5
+    (867, 867, 0),  # 5.2 / 4.9
+    (67, 133, 1),   # 3.7 / 7.8
+    (24, 47, 1),    # 3.5 / 6.9
+    (128, 231, 1),  # 3.6 / 4.8
+    (256, 405, 1),  # 4.1 / 4.8
+    (360, 539, 1),  # 4.1 / 5.6
+    (512, 765, 1),  # 4.2 / 5.0
+    (1000, 1215, 1),  # 4.6 / 5.2
+]
+
+
+@pytest.mark.parametrize("N,M,lines", ERRORS)
+def test_rule_by_error(ft, N, M, lines):
+    assert ft._lib.ftamd_grid_lines(N, M, 0) == lines
 
 
 @pytest.mark.parametrize("N,M,disk,lines", SIZES)
@@ -51,8 +75,8 @@ def test_hipfft_grids(ft, which):
     import torch
     geo = which.split("_")[0]
     rho = 0.4 if geo == "annulus" else None
-    for N, M in ((160, 315), (2187, 63)):
-        assert ft._lib.ftamd_grid_lines(N, M, geo == "disk") == (N == 160 and geo == "disk")
+    for N, M in ((60, 119), (2187, 63)):
+        assert ft._lib.ftamd_grid_lines(N, M, geo == "disk") == 0
         X = np.asfortranarray(np.random.default_rng(N + M).standard_normal((N, M)))
         for trans in ("N", "T"):
             syn = which.endswith("synthesis") == (trans == "N")
