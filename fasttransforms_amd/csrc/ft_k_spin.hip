@@ -181,10 +181,12 @@ __device__ void sweep(const Args &a, const Column &lq, const Column &cq, int jl,
         if (lvalid && t >= 0 && t <= RL)
             lA[(long long)(DIR == 0 ? RL - t : t) * a.row_stride] = sh.rows[S][lcol * PITCH + lk];
     };
-    for (int g = 0; g < rounds; g += 2) {
+    int g = 0;  // (the odd round out of the loop: a branch in it costs 2 % at n = 512)
+    for (; g + 1 < rounds; g += 2) {
         round(g, v0);
-        if (g + 1 < rounds) round(g + 1, v1);
+        round(g + 1, v1);
     }
+    if (g < rounds) round(g, v0);
     __threadfence_block();  // the next sweep's loads take rows that other lanes stored
     __syncthreads();
 }
