@@ -174,8 +174,10 @@ def _rows(kind, precision, direction, batch, found):
             out.append(row)
         lo = hi + 1
     if hi < NMAX_INT:
-        pipe = _best([r for r in found[-1][1] if r["cand"][0] == "pipeline"])
-        out.append(_row(kind, precision, direction, batch, lo, NMAX_INT, pipe["cand"]))
+        # of shapes that tie, more sequences a wave (disk n = 11500, M = 501: 8 3.56 ms, 4 3.69)
+        pipe = [r for r in found[-1][1] if r["cand"][0] == "pipeline"]
+        near = [r for r in pipe if r["ms"] is not None and r["ms"] <= 1.03 * _best(pipe)["ms"]]
+        out.append(_row(kind, precision, direction, batch, lo, NMAX_INT, max(near, key=lambda r: r["cand"][1])["cand"]))
     return out
 
 
