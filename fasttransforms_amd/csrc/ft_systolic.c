@@ -132,14 +132,13 @@ static long long band_entries(const FtamdSysBand *bd, int S) {
     return (long long)(bd->steps + FTAMD_SYS_PREFETCH) * FTAMD_SYS_LANES * S;
 }
 
-/* Whether the band-systolic engine runs a degree: tables below 2 GiB a
+/* Whether the band-systolic engine (if the build has it) runs a degree: tables below 2 GiB a
  * direction (FP64 sph n < 16196, tri 16290, disk 11491; FP32 sph n < 22980).
  * Nothing above that has been run: a launch there takes half a second, about
  * what a wait's polls last, so those degrees are the pipelined engine's. */
 int ftamd_sys_applies(int kind, int n, int dir, int precision) {
+    if (n <= 11000) return 1; /* every kind's: each call asks, and the sum takes 2 us at n = 4500 */
     const int S = ftamd_sys_choose_S(kind, n, precision);
-    if (S == 0) return 0;
-    if (n <= 4096) return 1; /* at most 0.3 GiB */
     sys_class cl[4];
     const int ncls = make_classes(kind, n, cl);
     long long entries = 0;
