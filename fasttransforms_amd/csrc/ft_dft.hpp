@@ -247,8 +247,9 @@ __device__ __forceinline__ bool cos_order(int q, int mode) { return mode == 3 ||
 // the passes (1800 FP64 instructions a thread and four exchanges, an LDS write
 // of 16 bytes a lane taking 13 clocks of the CU) take 10 of a phi launch's 28
 // us at n = 1024 (1024 x 2047), the rows' 16-byte pieces and the launch the
-// rest; theta (20 us) is its 34 MB and the launch.  Memory is read and written
-// once.  Workgroups go to XCDs in contiguous runs of lines, so that the
+// rest; theta (18 us) is its 34 MB and the launch.  At L = 8192
+// one workgroup is on a CU, 0.09 us a phi line and 0.16 a theta line (which
+// ftamd_grid_lines counts in).  Memory is read and written once.  Workgroups go to XCDs in contiguous runs of lines, so that the
 // 128-byte lines of memory that 4 to 8 neighbouring rows share stay in one L2.
 template <int LOGL, bool CHIRP>
 __global__ void __launch_bounds__(Shape<LOGL>::THREADS) lines_kernel(FtamdLines a) {

@@ -97,10 +97,10 @@ void ftamd_choose(int kind, int precision, int dir, int batch, int n, ftamd_choi
     const int found = ftamd_tuned_lookup(kind, precision, dir, batch, n, &te, &tm, &tL, &tW, &tg);
     const int ke = KNOB_GET(g_engine), km = KNOB_GET(g_sys_maxpart), kL = KNOB_GET(g_L), kW = KNOB_GET(g_W),
               kg = KNOB_GET(g_wg_per_cu);
-    /* built-in: the band-systolic engine for single transforms, the pipelined
-     * one for batches (many short chains leave the systolic one's CUs idle),
-     * whole chains of up to 16 bands, L 4, W 16, batches at 2 workgroups per
-     * CU (512 sph transforms of degree 32..1018: 9.9 ms capped, 10.4 ms not) */
+    /* without a table's row (another architecture, or the table switched off):
+     * the band-systolic engine for single transforms, the pipelined one for
+     * batches, which needs the largest plan's pairs alone, whole chains of up to
+     * 16 bands, L 4, W 16, batches at 2 workgroups per CU */
     c->forced = ke != FT_GPU_ENGINE_AUTO;
     c->engine = c->forced ? ke : found ? te : (batch ? FT_GPU_ENGINE_PIPELINE : FT_GPU_ENGINE_SYSTOLIC);
     if (!c->forced && c->engine == FT_GPU_ENGINE_SYSTOLIC && !ftamd_sys_applies(kind, n, dir, precision))
@@ -1848,10 +1848,10 @@ static int batch_cache_store(ft_batch_cache *B, ft_schedule *S, const ft_rotatio
     B->engine = engine;
     return FTAMD_OK;
 }
-/* Validates a batch and uploads the largest plan's table; *big gets that plan. */
 /* Validates a batch: plans of one family and one set of parameters (their
  * tables are one closed form), each of the kind's geometry with a valid
- * width.  Sets *geo and *layout of the kind and *big, the largest plan. */
+ * width.  Sets *geo and *layout of the kind and *big, the largest plan, whose
+ * table it uploads. */
 static int batch_check(const ft_rotation_plan *const *plans, int kind, int direction, int precision,
                        void *const *dA, const int *M, int count, int *geo, int *layout, ft_rotation_plan **big) {
     if (!plans || !dA || !M || count < 0 || (direction != 0 && direction != 1) || (precision != 0 && precision != 1))
@@ -2002,8 +2002,8 @@ static int batch_build_sys(const ft_rotation_plan *const *plans, int kind, int l
 
 /* Builds the schedule of a validated batch on the engine the tuning table
  * (or the caller) names.  256 sph transforms of degree 32 .. 1024 hi2lo in
- * FP64 take 3.8 ms band-systolic and 4.4 ms pipelined, disk ones 14.3 and 12.7
- * (long chains in several parts). */
+ * FP64 take 3.7 ms band-systolic and 4.4 ms pipelined, disk ones 14.1 and 12.7
+ * (long chains in several parts); 64 to 2896 17.7 and 15.8, 60 and 57. */
 static int batch_build(const ft_rotation_plan *const *plans, int kind, int layout, int direction, int precision,
                        void *const *dA, const int *M, int count, ft_rotation_plan *big, const ftamd_choice *ch,
                        ft_schedule **out) {

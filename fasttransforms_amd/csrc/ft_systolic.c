@@ -96,8 +96,8 @@ void ftamd_sys_tables_free(ft_sys_tables *T) {
     free(T);
 }
 
-/* Sequences per band lane of the plan's tables: 2, or 4 where the build has
- * no S = 2 engine for the precision (0 if neither). */
+/* Sequences per band lane of the plan's tables: 2 (or 4, should a build have
+ * only that engine for the precision; 0 if neither). */
 int ftamd_sys_choose_S(int kind, int n, int precision) {
     (void)kind;
     (void)n;
@@ -601,12 +601,14 @@ int ftamd_sys_assign(const FtamdSysChain *ch, int nch, const FtamdSysBand *bands
     /* A slot's list, in which a part that waits holds up those after it: the
      * first parts of split chains, whole chains, then the later parts in the
      * order of their place in the chain, whose rows are then there or on their
-     * way (FP64 against the order of the chains: sph n = 2047 lo2hi 1720 -> 980
-     * us, hi2lo 1140 -> 960; n = 1300 480 -> 333, 350 -> 300).  But hi2lo's
-     * parts grow along the chain, and the third ones, the longest and the
-     * longest waiting, would end last: with three parts or more it keeps the
-     * order of the chains (tri n = 1400 hi2lo 537 us against 600, n = 2048 1370
-     * against 1770). */
+     * way.  Against the order of the chains, us a launch, launches back to back,
+     * both sides in turn on one card (cards differ by 15 %): sph n = 2047 lo2hi
+     * 1708 -> 959, hi2lo 1128 -> 958; n = 1300 470 -> 300, 325 -> 269; tri n =
+     * 1400 lo2hi 827 -> 492; disk n = 1024 lo2hi 1014 -> 535.  But hi2lo's parts
+     * grow along the chain, and the third ones, the longest and the longest
+     * waiting, would end last: with three parts or more it keeps the order of
+     * the chains (tri n = 1400 hi2lo 537 us against 600, n = 2048 1370 against
+     * 1770). */
     int parts = 1;
     for (int c = 0, part = 0; c < nch; c++) {
         part = ch[c].split_in >= 0 ? part + 1 : 0;

@@ -318,7 +318,8 @@ struct Engine {
     // of the counters.  (sph hi2lo n = 1024, 1024 x 2047 FP64, with the copy
     // of the coefficients before it: 170 -> 142 us; FP32 lo2hi n = 733: 89 ->
     // 67 us, against selects per step, an LDS round trip per wait and the
-    // first band's rows through registers.  A step takes a lone wave about 190
+    // first band's rows through registers; the kernel alone under the
+    // profiler 192 -> 153.  A step takes a lone wave about 190
     // clocks, 22 of its instructions on the vector ALU; with four waves on a
     // SIMD the ALU bounds it.)
     template <int MASK, int END, bool LINK>

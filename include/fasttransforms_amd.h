@@ -525,12 +525,12 @@ int ft_gpu_tuning_table(int *rows, int cap);
 int ft_gpu_tuned_choice(int kind, int precision, int direction, int batch, int n, int *choice);
 
 /* Engine of the whole-matrix executors (no reference counterpart; for tests
- * and measurements): FT_GPU_ENGINE_AUTO (default) runs the band-systolic
- * engine wherever the build has it for the precision, the pipelined engine
- * elsewhere; FT_GPU_ENGINE_PIPELINE and FT_GPU_ENGINE_SYSTOLIC force one (the
- * latter fails with FT_GPU_EINVAL where it does not apply).  Batches run the
- * pipelined engine unless the systolic one is forced; single-vector kernels
- * always run the pipelined engine. */
+ * and measurements): FT_GPU_ENGINE_AUTO (default) runs the engine the tuning
+ * table names for the shape, single or batch, the pipelined one where the
+ * band-systolic engine does not apply (its tables would reach 2 GiB: FP64
+ * degrees from 16196 on, the disk's from 11491); FT_GPU_ENGINE_PIPELINE and
+ * FT_GPU_ENGINE_SYSTOLIC force one (the latter fails with FT_GPU_EINVAL where
+ * it does not apply).  Single-vector kernels always run the pipelined engine. */
 enum { FT_GPU_ENGINE_AUTO = 0, FT_GPU_ENGINE_PIPELINE = 1, FT_GPU_ENGINE_SYSTOLIC = 2 };
 int ft_gpu_set_engine(int engine);
 
