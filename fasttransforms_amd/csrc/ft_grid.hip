@@ -493,7 +493,7 @@ extern "C" int ftamd_grid_lines(int N, int M, int disk) {
     const int other = rest(N) * rest(M);
     if (other > 1) return 1;
     const int pn = ftamd_dft_points(N), pm = ftamd_dft_points(M);
-    if (N <= 256 && M <= 256) return N >= 128 && pn == N;
+    if (N <= 256 && M <= 256) return N == 1 || M == 1 || (N >= 128 && pn == N);
     const double lines = 0.9 * log2((double)pn) + 0.68 * log2((double)pm) - (pn == N ? 1.9 : 0.15);
     if (lines > 0.83 * hip) return 0;
     if (most > 7) return 1;

@@ -32,6 +32,7 @@ SIZES = [
     (2250, 63, 1, 0),    # 53.6 / 42.1
     (1000, 1323, 1, 1),  # 65.6 / 78.8
     (4097, 63, 0, 0), (63, 4097, 0, 0),  # longer than the lines
+    (1, 1, 0, 1), (1, 9, 0, 1), (9, 1, 0, 1),  # nothing to transform one way
 ]
 
 
@@ -70,13 +71,13 @@ def test_rule(ft, N, M, disk, lines):
 @pytest.mark.gpu
 @pytest.mark.parametrize("which", ["sph_synthesis", "sphv_analysis", "annulus_synthesis", "disk_synthesis",
                                    "disk_analysis"])
-def test_hipfft_grids(ft, which):
+def test_hipfft_and_shortest_grids(ft, which):
     import oracle as O
     import torch
     geo = which.split("_")[0]
     rho = 0.4 if geo == "annulus" else None
-    for N, M in ((60, 119), (2187, 63)):
-        assert ft._lib.ftamd_grid_lines(N, M, geo == "disk") == 0
+    for N, M in ((60, 119), (2187, 63), (2, 3), (1, 1), (1, 9), (2, 1)):
+        assert ft._lib.ftamd_grid_lines(N, M, geo == "disk") == (N == 1 or M == 1)
         X = np.asfortranarray(np.random.default_rng(N + M).standard_normal((N, M)))
         for trans in ("N", "T"):
             syn = which.endswith("synthesis") == (trans == "N")
